@@ -1,4 +1,4 @@
-// ar_gemm.hip -- MFMA GEMMs for gfx950: the reference's three linear kernels
+// ar_gemm.hip -- MFMA GEMMs for gfx950 with bf16 operands: the reference's three linear kernels
 // linear_fwd (NT, ops.mojo:110-203), linear_bwd_dx (NN, ops.mojo:870-950) and
 // linear_bwd_dw (TN, ops.mojo:953-1033), and the Muon Polar-Express products
 // that reuse them (optimizer.mojo:288-336).
@@ -13,15 +13,13 @@
 //
 // Design (CDNA4):
 //   * 256 threads = 4 wave64s, block tile 128x128, each wave a 64x64 quadrant
-//     computed as 2x2 MFMA 32x32 tiles (v_mfma_f32_32x32x16_bf16 for bf16
-//     compute, v_mfma_f32_32x32x2_f32 for exact fp32 compute).
+//     computed as 2x2 MFMA 32x32 tiles (v_mfma_f32_32x32x16_bf16); fp32 compute
+//     has its own kernel (ar_gemm_f32.hip).
 //   * K-major operands are staged through LDS in [row][k] layout (k
 //     contiguous, 16-byte padded rows) so every MFMA fragment is one
-//     ds_read_b128 (bf16) or ds_read_b32 (fp32).  With bf16 compute an
-//     MN-major operand stays in its natural [k][row] layout (16-byte loads
-//     and stores, chunks XOR-swizzled by k) and each fragment is two
-//     ds_read_b64_tr_b16 transpose reads; with fp32 compute it is transposed
-//     in registers on the way in.
+//     ds_read_b128.  An MN-major operand stays in its natural [k][row] layout
+//     (16-byte loads and stores, chunks XOR-swizzled by k) and each fragment is
+//     two ds_read_b64_tr_b16 transpose reads.
 //   * The epilogue stages each wave's accumulators through LDS and writes C
 //     (and reads the epilogue operand) as row-contiguous 4-wide vectors.
 //   * Two LDS stages; the next k-tile's global loads are issued before the
@@ -85,9 +83,7 @@ using TileL = Tile<256, 256, 2, 4>;
 enum Epi { EPI_STORE = 0, EPI_ACCUM = 1, EPI_PARTIAL = 2, EPI_ADD = 3, EPI_RELU2 = 4, EPI_SOFTCAP = 5,
            EPI_RELU2_BWD = 6, EPI_AXPBY = 7, EPI_QKV = 8, EPI_DOUT_D = 9 };
 
-template <bool BF16> struct Mfma;
-
-template <> struct Mfma<true> {
+struct Mfma {
     using LT = bf16;
     static constexpr int BK = 64, KS = 16, LDK = BK + 8, CW = 8;
     using Frag = bf16x8;
@@ -96,17 +92,6 @@ template <> struct Mfma<true> {
         return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
     }
     __device__ static int lane_k(int lane) { return (lane >> 5) * 8; }
-};
-
-template <> struct Mfma<false> {
-    using LT = float;
-    static constexpr int BK = 32, KS = 2, LDK = BK + 4, CW = 4;
-    using Frag = float;
-    __device__ static Frag frag(const LT* p) { return *p; }
-    __device__ static f32x16 mma(Frag a, Frag b, f32x16 c) {
-        return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
-    }
-    __device__ static int lane_k(int lane) { return lane >> 5; }
 };
 
 // Row of accumulator element v (0..15) of a 32x32 MFMA tile held by `lane`;
@@ -192,21 +177,17 @@ __device__ __forceinline__ void vzero(T (&dst)[N]) {
 // Global -> register -> LDS tile loader for one operand (ROWS x BK tile).
 //   K-major (KMAJ): LDS [row][k], rows padded to ldk, one 16-byte chunk of
 //     CW k-values per item.
-//   MN-major, bf16 compute (TR): LDS holds the natural [k][row] tile (ROWS
-//     bf16 per k, 16-byte chunks XOR-swizzled by tr_swz(k)); the MFMA
-//     fragments are read with ds_read_b64_tr_b16 (tr_frag).
-//   MN-major, fp32 compute: (k x 4-row) blocks transposed in registers into
-//     the [row][k] layout.
+//   MN-major (TR): LDS holds the natural [k][row] tile (ROWS bf16 per k,
+//     16-byte chunks XOR-swizzled by tr_swz(k)); the MFMA fragments are read
+//     with ds_read_b64_tr_b16 (tr_frag).
 __device__ __forceinline__ int tr_swz(int k) { return 4 * (k & 3); }
 
 template <typename TG, typename LT, bool KMAJ, int ROWS, int BK, int CW, int kThreads>
 struct TileLoader {
-    static constexpr bool TR = !KMAJ && sizeof(LT) == 2;
-    static constexpr int MW = 4;  // rows per MN-major item (fp32 compute)
-    static constexpr int NPASS = KMAJ ? (ROWS * BK / CW) / kThreads
-                                      : (TR ? (BK * ROWS / 8) / kThreads : ((BK / CW) * (ROWS / MW)) / kThreads);
-    static_assert(NPASS >= 1, "tile too small for the block");
-    static constexpr int PER = KMAJ ? CW : (TR ? 8 : CW * MW);  // TG values per pass
+    static constexpr bool TR = !KMAJ;
+    static constexpr int NPASS = (ROWS * BK / CW) / kThreads;
+    static_assert(NPASS >= 1 && CW == 8, "tile too small for the block");
+    static constexpr int PER = CW;  // TG values per pass
     TG v[NPASS][PER];
 
     // g: operand base; ld: row stride of the stored matrix; rows: extent of
@@ -228,26 +209,13 @@ struct TileLoader {
                 } else {
                     vzero(v[p]);
                 }
-            } else if constexpr (TR) {
+            } else {
                 const int item = p * kThreads + tid;
                 const int k = item / (ROWS / 8), c = item % (ROWS / 8);
                 const int lc = c ^ tr_swz(k);
                 const int64_t gk = k0 + k, gr = row0 + lc * 8;
                 if (gr < rows && gk < kend) vload(v[p], g + gk * ld + gr);
                 else vzero(v[p]);
-            } else {
-                const int item = p * kThreads + tid;
-                const int mg = item % (ROWS / MW), kg = item / (ROWS / MW);
-                const int64_t gr = row0 + mg * MW;
-#pragma unroll
-                for (int j = 0; j < CW; ++j) {
-                    const int64_t gk = k0 + kg * CW + j;
-                    TG tmp[MW];
-                    if (gr < rows && gk < kend) vload(tmp, g + gk * ld + gr);
-                    else vzero(tmp);
-#pragma unroll
-                    for (int i = 0; i < MW; ++i) v[p][j * MW + i] = tmp[i];
-                }
             }
         }
     }
@@ -263,23 +231,12 @@ struct TileLoader {
 #pragma unroll
                 for (int i = 0; i < CW; ++i) out[i] = (LT)to_f32(v[p][i]);
                 *reinterpret_cast<uint4*>(lds + r * ldk + kc) = *reinterpret_cast<const uint4*>(out);
-            } else if constexpr (TR) {
+            } else {
                 const int item = p * kThreads + tid;
                 LT out[8];
 #pragma unroll
                 for (int i = 0; i < 8; ++i) out[i] = (LT)to_f32(v[p][i]);
                 *reinterpret_cast<uint4*>(lds + item * 8) = *reinterpret_cast<const uint4*>(out);
-            } else {
-                const int item = p * kThreads + tid;
-                const int mg = item % (ROWS / MW), kg = item / (ROWS / MW);
-#pragma unroll
-                for (int i = 0; i < MW; ++i) {
-                    LT out[CW];
-#pragma unroll
-                    for (int j = 0; j < CW; ++j) out[j] = (LT)to_f32(v[p][j * MW + i]);
-                    *reinterpret_cast<uint4*>(lds + (mg * MW + i) * ldk + kg * CW) =
-                        *reinterpret_cast<const uint4*>(out);
-                }
             }
         }
     }
@@ -320,14 +277,14 @@ __device__ __forceinline__ void tile_coords(int64_t tiles_n, int64_t tiles_mn, i
     tn = r % tiles_n;
 }
 
-template <typename TA, typename TB, typename TC, bool AK, bool BKM, bool BF16, int EPI, typename TL>
+template <typename TA, typename TB, typename TC, bool AK, bool BKM, int EPI, typename TL>
 __global__ __launch_bounds__(TL::THREADS) void gemm_k(TC* C, const TA* A, const TB* B, int64_t M, int64_t N,
                                                       int64_t K, int64_t lda, int64_t ldb, int64_t ldc,
                                                       int64_t k_per_split, float* partial, int64_t batch,
                                                       int64_t sA, int64_t sB, int64_t sC, const void* aux,
                                                       void* aux_out, float cap, float beta) {
-    using MM = Mfma<BF16>;
-    using LT = typename MM::LT;
+    using MM = Mfma;
+    using LT = MM::LT;
     constexpr int BM = TL::BM, BN = TL::BN, TM = TL::TM, TN = TL::TN;
     constexpr int BK = MM::BK, LDK = MM::LDK, CW = MM::CW;
     extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -390,7 +347,7 @@ __global__ __launch_bounds__(TL::THREADS) void gemm_k(TC* C, const TA* A, const 
         const LT* b_base = sb + (wn * TL::WN + (lane & 31)) * LDK + MM::lane_k(lane);
 #pragma unroll
         for (int ks = 0; ks < BK / MM::KS; ++ks) {
-            typename MM::Frag fa[TM], fb[TN];
+            MM::Frag fa[TM], fb[TN];
 #pragma unroll
             for (int i = 0; i < TM; ++i) {
                 if constexpr (LA::TR) fa[i] = tr_frag<BM>(sa, wm * TL::WM + i * 32, ks, lane);
@@ -1221,11 +1178,10 @@ static void splitk_reduce(hipStream_t st, TC* C, const float* partial, int64_t M
                                                                                accumulate ? 1 : 0, batch, sC);
 }
 
-template <bool BF16, typename TL>
+template <typename TL>
 constexpr size_t lds_bytes() {
-    using MM = Mfma<BF16>;
     // K-major tiles are the larger layout (padded rows); TR tiles fit inside.
-    const size_t stages = (size_t)2 * (TL::BM + TL::BN) * MM::LDK * sizeof(typename MM::LT);
+    const size_t stages = (size_t)2 * (TL::BM + TL::BN) * Mfma::LDK * sizeof(Mfma::LT);
     const size_t strips = (size_t)(TL::THREADS / 64) * 32 * (TL::WN + 8) * sizeof(float);
     return stages > strips ? stages : strips;
 }
@@ -1234,9 +1190,8 @@ constexpr size_t lds_bytes() {
 
 namespace ar {
 
-template <bool BF16>
-static int64_t choose_splits(int64_t tiles, int64_t K, int64_t splits_req, int64_t& kps, int64_t target = 512) {
-    constexpr int BKt = Mfma<BF16>::BK;
+static int64_t choose_splits(int64_t tiles, int64_t K, int64_t splits_req, int64_t& kps, int64_t target = 512,
+                             int64_t BKt = Mfma::BK) {
     int64_t splits = splits_req;
     if (splits < 1) {
         // Aim for `target` workgroups when the reduction is long.
@@ -1251,7 +1206,7 @@ static int64_t choose_splits(int64_t tiles, int64_t K, int64_t splits_req, int64
 
 // Launches one GEMM in GEMM space: C[mo, no] (+)= sum_r A(mo, r) B(no, r).
 // epi: EPI_STORE / EPI_ACCUM select by `accumulate` when epi < 0.
-template <typename TA, typename TB, typename TC, bool AK, bool BKM, bool BF16, typename TL>
+template <typename TA, typename TB, typename TC, bool AK, bool BKM, typename TL>
 static int32_t gemm_launch_t(hipStream_t st, TC* C, const TA* A, const TB* B, int64_t M, int64_t N, int64_t K,
                              int64_t lda, int64_t ldb, int64_t ldc, bool accumulate, int64_t splits_req,
                              float* partial, const char* nm, int64_t batch, int64_t sA, int64_t sB, int64_t sC,
@@ -1260,12 +1215,12 @@ static int32_t gemm_launch_t(hipStream_t st, TC* C, const TA* A, const TB* B, in
     int64_t kps = 0;
     // one 256x256 workgroup per CU, two 128x128 ones
     const int64_t target = TL::BM == 256 ? 256 : 512;
-    const int64_t splits = epi >= 0 ? 1 : choose_splits<BF16>(tiles * batch, K, splits_req, kps, target);
-    if (epi >= 0) choose_splits<BF16>(tiles * batch, K, 1, kps);
-    const size_t lds = lds_bytes<BF16, TL>();
+    const int64_t splits = epi >= 0 ? 1 : choose_splits(tiles * batch, K, splits_req, kps, target);
+    if (epi >= 0) choose_splits(tiles * batch, K, 1, kps);
+    const size_t lds = lds_bytes<TL>();
     const unsigned grid = (unsigned)(tiles * splits * batch);
 #define AR_GK(E)                                                                                              \
-    gemm_k<TA, TB, TC, AK, BKM, BF16, E, TL><<<grid, TL::THREADS, lds, st>>>(C, A, B, M, N, K, lda, ldb, ldc, kps, \
+    gemm_k<TA, TB, TC, AK, BKM, E, TL><<<grid, TL::THREADS, lds, st>>>(C, A, B, M, N, K, lda, ldb, ldc, kps, \
                                                                             partial, batch, sA, sB, sC, aux,    \
                                                                             aux_out, cap, beta)
     if (epi >= 0) {
@@ -1471,17 +1426,17 @@ inline bool use_large(int64_t M, int64_t N, int64_t K, int64_t batch) {
     return t >= 256 || (K >= 16384 && t >= 4);
 }
 
-template <typename TA, typename TB, typename TC, bool AK, bool BKM, bool BF16>
+template <typename TA, typename TB, typename TC, bool AK, bool BKM>
 static int32_t gemm_launch(hipStream_t st, TC* C, const TA* A, const TB* B, int64_t M, int64_t N, int64_t K,
                            int64_t lda, int64_t ldb, int64_t ldc, bool accumulate, int64_t splits_req,
                            float* partial, const char* nm, int64_t batch = 1, int64_t sA = 0, int64_t sB = 0,
                            int64_t sC = 0, int epi = -1, const void* aux = nullptr, void* aux_out = nullptr,
                            float cap = 0.f, float beta = 0.f) {
     if (use_large(M, N, K, batch))
-        return gemm_launch_t<TA, TB, TC, AK, BKM, BF16, TileL>(st, C, A, B, M, N, K, lda, ldb, ldc, accumulate,
+        return gemm_launch_t<TA, TB, TC, AK, BKM, TileL>(st, C, A, B, M, N, K, lda, ldb, ldc, accumulate,
                                                                splits_req, partial, nm, batch, sA, sB, sC, epi, aux,
                                                                aux_out, cap, beta);
-    return gemm_launch_t<TA, TB, TC, AK, BKM, BF16, TileS>(st, C, A, B, M, N, K, lda, ldb, ldc, accumulate,
+    return gemm_launch_t<TA, TB, TC, AK, BKM, TileS>(st, C, A, B, M, N, K, lda, ldb, ldc, accumulate,
                                                            splits_req, partial, nm, batch, sA, sB, sC, epi, aux,
                                                            aux_out, cap, beta);
 }
@@ -1493,13 +1448,14 @@ static void gemm_space(int layout, int64_t M, int64_t N, int64_t K, int64_t& gm,
     else { gm = N; gn = K; gk = M; }
 }
 
-// Split count of gemm_k's automatic choice for a TN call.
+// Split count of gemm_k's automatic choice for a TN call, and the most that an
+// fp32 one may use (gemm_x3 takes what pays): scratch is sized with it.
 static int64_t gemm_k_splits(bool bf16, int64_t gm, int64_t gn, int64_t gk) {
     int64_t kps;
     const bool large = use_large(gm, gn, gk, 1);
     const int64_t tiles = large ? ((gm + 255) / 256) * ((gn + 255) / 256) : ((gm + 127) / 128) * ((gn + 127) / 128);
     const int64_t target = large ? 256 : 512;
-    return bf16 ? choose_splits<true>(tiles, gk, 0, kps, target) : choose_splits<false>(tiles, gk, 0, kps, target);
+    return choose_splits(tiles, gk, 0, kps, target, bf16 ? Mfma::BK : 32);
 }
 
 // Split count of a TN call: the persistent kernel's for the shapes it runs
@@ -1532,7 +1488,7 @@ int32_t gemm_batched_bf16(hipStream_t st, bool ak, bool bk, float* C, bf16* Cb, 
                           int64_t sA, int64_t sB, int64_t sC, const float* aux, float alpha, float beta) {
     const int epi = aux ? EPI_AXPBY : -1;
 #define AR_GB(AKv, BKv)                                                                                          \
-    gemm_launch<bf16, bf16, float, AKv, BKv, true>(st, C, A, B, M, N, K, lda, ldb, ldc, false, 1, nullptr,         \
+    gemm_launch<bf16, bf16, float, AKv, BKv>(st, C, A, B, M, N, K, lda, ldb, ldc, false, 1, nullptr,         \
                                                    "gemm_batched_bf16", batch, sA, sB, sC, epi, aux, Cb, alpha, beta)
     if (ak && bk) return AR_GB(true, true);
     if (ak && !bk) return AR_GB(true, false);
@@ -1545,13 +1501,12 @@ int32_t gemm_batched_f32(hipStream_t st, bool bf, bool ak, bool bk, float* C, co
                          int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldc, int64_t batch,
                          int64_t sA, int64_t sB, int64_t sC, const float* aux, float alpha, float beta) {
     const int epi = aux ? EPI_AXPBY : -1;
-#define AR_GB(AKv, BKv)                                                                                        \
-    (bf ? gemm_launch<float, float, float, AKv, BKv, true>(st, C, A, B, M, N, K, lda, ldb, ldc, false, 1, nullptr, \
-                                                           "gemm_batched", batch, sA, sB, sC, epi, aux, nullptr, \
-                                                           alpha, beta)                                       \
-        : gemm_launch<float, float, float, AKv, BKv, false>(st, C, A, B, M, N, K, lda, ldb, ldc, false, 1, nullptr, \
-                                                            "gemm_batched", batch, sA, sB, sC, epi, aux, nullptr, \
-                                                            alpha, beta))
+    if (!bf)
+        return gemm_x3(st, ak, bk, C, A, B, M, N, K, lda, ldb, ldc, 1, nullptr, aux, alpha, beta, batch, sA, sB, sC,
+                       nullptr, "gemm_batched");
+#define AR_GB(AKv, BKv)                                                                                           \
+    gemm_launch<float, float, float, AKv, BKv>(st, C, A, B, M, N, K, lda, ldb, ldc, false, 1, nullptr, "gemm_batched", \
+                                               batch, sA, sB, sC, epi, aux, nullptr, alpha, beta)
     if (ak && bk) return AR_GB(true, true);
     if (ak && !bk) return AR_GB(true, false);
     if (!ak && !bk) return AR_GB(false, false);
@@ -1579,14 +1534,14 @@ static int32_t gemm_typed(hipStream_t st, int layout, TC* C, const TX* X, const 
         }
     }
     if (layout == 0)
-        return gemm_launch<TX, TW, TC, true, true, true>(st, C, X, W, M, N, K, K, K, N, accumulate, 1, nullptr,
+        return gemm_launch<TX, TW, TC, true, true>(st, C, X, W, M, N, K, K, K, N, accumulate, 1, nullptr,
                                                          "linear_fwd");
     if (layout == 1)
-        return gemm_launch<TX, TW, TC, true, false, true>(st, C, X, W, M, K, N, N, K, K, accumulate, 1, nullptr,
+        return gemm_launch<TX, TW, TC, true, false>(st, C, X, W, M, K, N, N, K, K, accumulate, 1, nullptr,
                                                           "linear_bwd_dx");
     if (splits < 1)
         splits = gemm_auto_splits(2, true, std::is_same<TX, bf16>::value && std::is_same<TW, bf16>::value, M, N, K);
-    return gemm_launch<TX, TW, TC, false, false, true>(st, C, X, W, N, K, M, N, K, K, accumulate, splits, partial,
+    return gemm_launch<TX, TW, TC, false, false>(st, C, X, W, N, K, M, N, K, K, accumulate, splits, partial,
                                                        "linear_bwd_dw");
 }
 
@@ -1625,10 +1580,10 @@ int32_t gemm_epilogue(hipStream_t st, int layout, int epi, void* C, int c_bf16, 
                                                           epi, aux, aux_out, cap, "gemm_epilogue");
     }
 #define AR_GE(TX, TW, TC)                                                                                          \
-    (layout == 0 ? gemm_launch<TX, TW, TC, true, true, true>(st, (TC*)C, (const TX*)X, (const TW*)W, M, N, K, K, K, N, \
+    (layout == 0 ? gemm_launch<TX, TW, TC, true, true>(st, (TC*)C, (const TX*)X, (const TW*)W, M, N, K, K, K, N, \
                                                              false, 1, nullptr, "gemm_epilogue", 1, 0, 0, 0, epi, aux, \
                                                              aux_out, cap)                                         \
-                 : gemm_launch<TX, TW, TC, true, false, true>(st, (TC*)C, (const TX*)X, (const TW*)W, M, K, N, N, K,  \
+                 : gemm_launch<TX, TW, TC, true, false>(st, (TC*)C, (const TX*)X, (const TW*)W, M, K, N, N, K,  \
                                                               K, false, 1, nullptr, "gemm_epilogue", 1, 0, 0, 0, epi, \
                                                               aux, aux_out, cap))
     if (x_bf16 && w_bf16 && c_bf16) return AR_GE(bf16, bf16, bf16);
@@ -1642,37 +1597,38 @@ int32_t gemm_epilogue(hipStream_t st, int layout, int epi, void* C, int c_bf16, 
 int32_t gemm_f32_add(hipStream_t st, bool bf, float* C, const float* X, const float* W, const float* R, int64_t M,
                      int64_t N, int64_t K) {
     if (bf)
-        return gemm_launch<float, float, float, true, true, true>(st, C, X, W, M, N, K, K, K, N, false, 1, nullptr,
-                                                                  "linear_fwd_add", 1, 0, 0, 0, EPI_ADD, R, nullptr,
-                                                                  0.f);
-    return gemm_launch<float, float, float, true, true, false>(st, C, X, W, M, N, K, K, K, N, false, 1, nullptr,
-                                                               "linear_fwd_add", 1, 0, 0, 0, EPI_ADD, R, nullptr, 0.f);
+        return gemm_launch<float, float, float, true, true>(st, C, X, W, M, N, K, K, K, N, false, 1, nullptr,
+                                                            "linear_fwd_add", 1, 0, 0, 0, EPI_ADD, R, nullptr, 0.f);
+    return gemm_x3(st, true, true, C, X, W, M, N, K, K, K, N, 1, nullptr, R, 1.f, 1.f, 1, 0, 0, 0, nullptr,
+                   "linear_fwd_add");
 }
 
 int32_t gemm_f32(hipStream_t st, int layout, bool bf, float* C, const float* X, const float* W, int64_t M, int64_t N,
                  int64_t K, bool accumulate, int64_t splits, float* partial) {
-    if (layout == 0) {
-        if (bf)
-            return gemm_launch<float, float, float, true, true, true>(st, C, X, W, M, N, K, K, K, N, accumulate, 1,
-                                                                      nullptr, "linear_fwd");
-        return gemm_launch<float, float, float, true, true, false>(st, C, X, W, M, N, K, K, K, N, accumulate, 1,
-                                                                   nullptr, "linear_fwd");
+    static const char* const names[3] = {"linear_fwd", "linear_bwd_dx", "linear_bwd_dw"};
+    if (layout == 2 && splits < 1) splits = gemm_auto_splits(2, bf, false, M, N, K);
+    if (!bf) {
+        int64_t gm, gn, gk, used = 1;
+        gemm_space(layout, M, N, K, gm, gn, gk);
+        // row strides of X, W and C as stored: reduction- or output-contiguous
+        const int64_t lda = layout == 0 ? K : N, ldb = K, ldc = layout == 0 ? N : K;
+        int32_t r = gemm_x3(st, layout != 2, layout == 0, C, X, W, gm, gn, gk, lda, ldb, ldc, splits, partial,
+                            accumulate ? C : nullptr, 1.f, 1.f, 1, 0, 0, 0, &used, names[layout]);
+        if (r == AR_OK && used > 1) {
+            splitk_reduce<float>(st, C, partial, gm, gn, ldc, used, accumulate, 1, 0);
+            r = check_launch(names[layout]);
+        }
+        return r;
     }
-    if (layout == 1) {
-        // GEMM (mo=M, no=K, r=N): A = dY [M][N] K-major, B(no=k, r=n) = W[n][k] MN-major.
-        if (bf)
-            return gemm_launch<float, float, float, true, false, true>(st, C, X, W, M, K, N, N, K, K, accumulate, 1,
-                                                                       nullptr, "linear_bwd_dx");
-        return gemm_launch<float, float, float, true, false, false>(st, C, X, W, M, K, N, N, K, K, accumulate, 1,
-                                                                    nullptr, "linear_bwd_dx");
-    }
+    if (layout == 0)
+        return gemm_launch<float, float, float, true, true>(st, C, X, W, M, N, K, K, K, N, accumulate, 1, nullptr,
+                                                            names[0]);
+    if (layout == 1)  // GEMM (mo=M, no=K, r=N): A = dY [M][N] K-major, B(no=k, r=n) = W[n][k] MN-major.
+        return gemm_launch<float, float, float, true, false>(st, C, X, W, M, K, N, N, K, K, accumulate, 1, nullptr,
+                                                             names[1]);
     // TN: GEMM (mo=N, no=K, r=M): A(mo=n, r=m) = dY[m][n] MN-major, B(no=k, r=m) = X[m][k] MN-major.
-    if (splits < 1) splits = gemm_auto_splits(2, bf, false, M, N, K);
-    if (bf)
-        return gemm_launch<float, float, float, false, false, true>(st, C, X, W, N, K, M, N, K, K, accumulate,
-                                                                    splits, partial, "linear_bwd_dw");
-    return gemm_launch<float, float, float, false, false, false>(st, C, X, W, N, K, M, N, K, K, accumulate, splits,
-                                                                 partial, "linear_bwd_dw");
+    return gemm_launch<float, float, float, false, false>(st, C, X, W, N, K, M, N, K, K, accumulate, splits, partial,
+                                                          names[2]);
 }
 
 }  // namespace ar
@@ -1695,8 +1651,8 @@ static inline bool overlaps(const void* a, size_t abytes, const void* b, size_t 
     return pa < pb + bbytes && pb < pa + abytes;
 }
 
-// The matrix-core kernels take dimensions in multiples of 8 and 16-byte
-// aligned operands.  Other calls run the same kernels on zero-padded copies
+// The bf16-compute kernels take dimensions in multiples of 8 and 16-byte
+// aligned operands.  Other bf16 calls (and fp32 ones with an extent below 8) run the same kernels on zero-padded copies
 // in the workspace (the padding adds zero products only) and copy the valid
 // region back: the tail path of the reference's bounds-checked tiles
 // (ops.mojo:150-168).
@@ -1816,7 +1772,11 @@ static int32_t linear_call(ar_stream_t s, int layout, bool bf, float* C, const f
         ws = (char*)ar::workspace(S(s), need, &st);
         if (!ws) return st;
     }
-    if (!gemm_direct(C, X, W, M, N, K)) return gemm_padded(S(s), layout, bf, C, X, W, M, N, K, ws);
+    // The fp32 kernel takes odd sizes and 4-byte alignment as they are; only an
+    // extent below 8 still goes through the padded copies.  (The workspace of
+    // the padded path stays a condition of the call; it covers the partials.)
+    const bool as_is = gemm_direct(C, X, W, M, N, K) || (!bf && M >= 8 && N >= 8 && K >= 8);
+    if (!as_is) return gemm_padded(S(s), layout, bf, C, X, W, M, N, K, ws);
     const float* src = X;
     if (layout == 1 && overlaps(C, cb, X, (size_t)M * N * 4)) {
         // model.mojo:906 calls this in place; read all of dY first (copy).
@@ -1827,7 +1787,8 @@ static int32_t linear_call(ar_stream_t s, int layout, bool bf, float* C, const f
     int64_t splits = 1;
     float* partial = nullptr;
     if (layout == 2) {
-        splits = ar::gemm_auto_splits(2, bf, false, M, N, K);
+        splits = gemm_direct(C, X, W, M, N, K) ? ar::gemm_auto_splits(2, bf, false, M, N, K)
+                                               : ar::gemm_auto_splits(2, bf, false, r8(M), r8(N), r8(K));
         if (splits > 1) partial = (float*)ws;
     }
     return ar::gemm_f32(S(s), layout, bf, C, src, W, M, N, K, layout == 2, splits, partial);

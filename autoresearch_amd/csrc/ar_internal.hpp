@@ -25,7 +25,17 @@ int32_t gemm_f32(hipStream_t st, int layout, bool bf16, float* C, const float* X
 // the add in fp32 exactly as a separate residual add does it (R may alias C).
 int32_t gemm_f32_add(hipStream_t st, bool bf16, float* C, const float* X, const float* W, const float* R, int64_t M,
                      int64_t N, int64_t K);
-// Same, with each operand stored as bf16 (flag set) or fp32; bf16 compute.
+// fp32 products on the bf16 matrix cores by three-term splitting
+// (ar_gemm_f32.hip), in GEMM space: C_b[m, n] = sum_r A_b(m, r) B_b(n, r), or
+// alpha times that + beta aux_b (aux laid out as C; may be C).  With partial
+// set the reduction may be split up to max_splits ways: then *splits > 1 and
+// partial holds [batch][splits][M][N] for the caller to add (aux not applied).
+bool gemm_x3_ok(bool ak, bool bk, int64_t M, int64_t N, int64_t K);
+int32_t gemm_x3(hipStream_t st, bool ak, bool bk, float* C, const float* A, const float* B, int64_t M, int64_t N,
+                int64_t K, int64_t lda, int64_t ldb, int64_t ldc, int64_t max_splits, float* partial,
+                const float* aux, float alpha, float beta, int64_t batch, int64_t sA, int64_t sB, int64_t sC,
+                int64_t* splits, const char* nm);
+// Same as gemm_f32, with each operand stored as bf16 (flag set) or fp32; bf16 compute.
 int32_t gemm_bf16io(hipStream_t st, int layout, void* C, int c_bf16, const void* X, int x_bf16, const void* W,
                     int w_bf16, int64_t M, int64_t N, int64_t K, bool accumulate, int64_t splits, float* partial);
 // NT (layout 0) / NN (layout 1) GEMM with a fused epilogue, bf16 compute:

@@ -235,11 +235,11 @@ int32_t muon_group_step(hipStream_t st, float* const* params, const float* const
     // Each iteration's combinations ride on the product before them:
     // Bm = cb A + cc (A A) in the A.A epilogue, and X' = ca X + (B X or X B)
     // in the last product's epilogue, written to the other of X / Y.
-    // A = X^T X (or X X^T) is symmetric bit for bit: entries (i, j) and
-    // (j, i) sum the same products in the same k order.  So is A A, and with
-    // it Bm.  A symmetric operand read as the B side of a product is read
-    // K-major (its own transpose), the GEMM's faster LDS path, with the same
-    // values in the same order.
+    // A = X^T X (or X X^T) is symmetric: entries (i, j) and (j, i) sum the same
+    // products in the same k order (bf16: equal bit for bit; fp32: to the
+    // rounding of the split's small terms, added in the other order).  So is
+    // A A, and with it Bm.  A symmetric operand read as the B side of a product is read
+    // K-major (its own transpose), the GEMM's faster LDS path.
     float* Xc = X;
     float* Yc = Y;
     ::ar::bf16* Xbc = Xb;
