@@ -1,6 +1,6 @@
 // ar_flash.hip -- flash attention for bf16-stored operands (the bf16 step):
 // forward (ops.mojo:244-323), dQ (ops.mojo:349-411) and dK/dV
-// (ops.mojo:414-480), same math and work split as ar_attention.hip, with the
+// (ops.mojo:414-480), same math as ar_attn_f32.hip, with the
 // data movement rebuilt around two gfx950 features:
 //
 //   * Natural tiles only.  Every streamed 64-row tile (K, V, Q, dO) sits in

@@ -2,15 +2,11 @@
 // linear_bwd_dw of ops.mojo:110-203, 870-950, 953-1033 and the fp32 Muon
 // products, optimizer.mojo:288-336) on the bf16 matrix cores, at fp32 accuracy.
 //
-// Each fp32 operand value is split exactly into three bf16 terms
-//   a = hi + mid + lo,  hi = bf16(a), mid = bf16(a - hi), lo = a - hi - mid
-// (8 significant bits each: 24 in all, and both differences are exact), and
+// Each operand value is split exactly into three bf16 terms (ar_split.hpp) and
 // the product is the sum of the six terms down to 2^-18 of the leading one,
-//   a b = lo hi + hi lo + mid mid + mid hi + hi mid + hi hi,
-// accumulated in fp32 (hi hi in one accumulator, the smaller terms in another);
-// the three dropped terms are below 2^-25 of it, less than half an fp32
-// rounding.  Six v_mfma_f32_32x32x16_bf16 do 16 k-values in 192 cycles where
-// eight v_mfma_f32_32x32x2_f32 take 512, and round the sum once instead of eight
+// accumulated in fp32: hi hi in one accumulator, the smaller terms in another.
+// Six v_mfma_f32_32x32x16_bf16 do 16 k-values in 192 cycles where eight
+// v_mfma_f32_32x32x2_f32 take 512, and round the sum once instead of eight
 // times: norm-wise error against fp64 1.3e-7 at 512^3 (N(0, 1) operands) where
 // the fp32 instruction gave 4.1e-7.
 //
@@ -25,6 +21,7 @@
 // Layout of a product (GEMM space): C[m, n] (+)= sum_r A(m, r) B(n, r), each
 // operand K-major (r contiguous) or MN-major (m / n contiguous).
 #include "ar_internal.hpp"
+#include "ar_split.hpp"
 
 #include <math.h>
 
@@ -67,44 +64,11 @@ struct X3Args {
     int batch;
 };
 
-// 16-byte unit slot of a staged K-major tile (U units per row): 16 rows of one
-// unit fill all 64 banks once.
-template <int U>
-__device__ __forceinline__ int kslot(int r, int c) {
-    static_assert(U == 4 || U == 8 || U == 16, "32-, 64- or 128-deep tiles");
-    return U == 4 ? r * 4 + (c ^ ((r >> 2) & 3)) : U == 8 ? r * 8 + (c ^ ((r >> 1) & 7)) : r * 16 + (c ^ (r & 15));
-}
 // Chunk swizzle of a staged MN-major tile [k][ROWS]: the four k-rows one
 // transpose read touches (64 bytes of each) fall into different quarters of the banks.
 template <int ROWS>
 __device__ __forceinline__ int mnswz(int k) {
     return ROWS >= 128 ? 4 * (k & 3) : ROWS == 64 ? 4 * ((k >> 1) & 1) : 0;
-}
-
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-
-// x = hi + mid + lo for values e, e + 1 of an item.  The two exact differences are dot products
-// of the rounded pair with (-1, 0) / (0, -1): one v_dot2_f32_bf16 where a
-// widening and a subtraction would be two, 3.5 VALU per value instead of 5.5.
-// The constants go through scalar registers: as an inline constant -1.0 the
-// hardware reads the fp32 pattern, whose low half is zero.
-__device__ __forceinline__ void split2(float x0, float x1, int e, bf16x8& hi, bf16x8& mid, bf16x8& lo) {
-    unsigned c0 = 0x0000BF80u, c1 = 0xBF800000u;
-    asm("" : "+s"(c0), "+s"(c1));
-    const bf16x2 s0 = __builtin_bit_cast(bf16x2, c0), s1 = __builtin_bit_cast(bf16x2, c1);
-    bf16x2 h, m;
-    h[0] = (bf16)x0;
-    h[1] = (bf16)x1;
-    const float r0 = __builtin_amdgcn_fdot2_f32_bf16(h, s0, x0, false);
-    const float r1 = __builtin_amdgcn_fdot2_f32_bf16(h, s1, x1, false);
-    m[0] = (bf16)r0;
-    m[1] = (bf16)r1;
-    hi[e] = h[0];
-    hi[e + 1] = h[1];
-    mid[e] = m[0];
-    mid[e + 1] = m[1];
-    lo[e] = (bf16)__builtin_amdgcn_fdot2_f32_bf16(m, s0, r0, false);
-    lo[e + 1] = (bf16)__builtin_amdgcn_fdot2_f32_bf16(m, s1, r1, false);
 }
 
 // v[0..7] = v[s..7], then whatever was there (s < 8): a conditional move per

@@ -105,14 +105,13 @@ int32_t ve_gate_bwd(hipStream_t st, bf16* gx, float* gw, const float* ggate, con
                     const float* w, int64_t nt, int64_t nkv, int64_t gc, int64_t C, int64_t ldx, float* partial);
 constexpr int kGateMaxH = 16;
 
-// ---- attention (ar_attention.hip) ----
+// ---- attention (fp32: ar_attn_f32.hip) ----
 enum class AttnOp { FWD, DQ, DKV };
 // scale: the softmax scale; 0 = 1/sqrt(HD).  A caller that zero-pads rows
 // from a smaller head_dim to HD passes 1/sqrt of the unpadded head_dim.
-template <bool BF16, typename TIN>
-int32_t attn_dispatch(hipStream_t st, AttnOp op, float* o1, float* o2, const TIN* q, const TIN* k, const TIN* v,
-                      const TIN* dout, const float* lse, const float* dbuf, int64_t B, int64_t T, int64_t H,
-                      int64_t HD, int64_t window, float scale = 0.f);
+int32_t attn_f32(hipStream_t st, AttnOp op, float* o1, float* o2, const float* q, const float* k, const float* v,
+                 const float* dout, const float* lse, const float* dbuf, int64_t B, int64_t T, int64_t H, int64_t HD,
+                 int64_t window, float scale = 0.f);
 
 // bf16-stored operands (ar_flash.hip): q, k, v, dout bf16.  fp32 outputs
 // (may be null except LSE): FWD o1 = O, o2 = LSE; DQ o1 = dQ; DKV o1 = dK,

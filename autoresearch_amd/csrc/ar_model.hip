@@ -242,8 +242,7 @@ void attn_prof_end(ar_gpt* m, int e, AttnOp op, int64_t ws) {
 int32_t attention(ar_gpt* m, AttnOp op, float* o1, float* o2, const float* q, const float* k, const float* v,
                   const float* dout, const float* lse, const float* dbuf, int64_t ws) {
     const int e = prof_begin(m);
-    const int32_t r = attn_dispatch<false, float>(m->st, op, o1, o2, q, k, v, dout, lse, dbuf, m->B, m->T,
-                                                  m->c.n_head, m->c.head_dim, ws);
+    const int32_t r = attn_f32(m->st, op, o1, o2, q, k, v, dout, lse, dbuf, m->B, m->T, m->c.n_head, m->c.head_dim, ws);
     attn_prof_end(m, e, op, ws);
     return r;
 }
