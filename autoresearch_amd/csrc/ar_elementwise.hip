@@ -110,8 +110,50 @@ __global__ void relu2_bwd_k(float* dx, const float* dy, const float* x, int64_t 
 }
 
 // ---------------- K10 softcap ----------------
+// tanh(y) in few enough instructions that the pass stays HBM-bound (with the
+// library's tanhf and one value per lane it was bound by arithmetic: 67.1M
+// values 157 us, 92 here).  |y| <= 1: y + y^3 P(y^2), P a near-minimax
+// fit of (tanh(y) / y - 1) / y^2 (6e-10 relative); beyond: 1 - 2 / (e^(2 |y|)
+// + 1), with the roundings of the exponential's argument and of the sum
+// carried into the reciprocal's correction.  Both sides are computed and one
+// selected.  Largest error against 64 bits 0.89 ulp, mean 0.26 (tanhf's:
+// 1.40, 0.34).  2^inf = inf gives exactly +-1; a NaN takes the polynomial.
+__device__ __forceinline__ float tanh_pass(float y) {
+    const float z = y * y, a = fabsf(y);
+    float p = 0x1.ee50cep-14f;
+    p = fmaf(p, z, -0x1.b1af04p-11f);
+    p = fmaf(p, z, 0x1.90a7d2p-9f);
+    p = fmaf(p, z, -0x1.190ffep-7f);
+    p = fmaf(p, z, 0x1.64ca42p-6f);
+    p = fmaf(p, z, -0x1.b9f7c6p-5f);
+    p = fmaf(p, z, 0x1.111040p-3f);
+    p = fmaf(p, z, -0x1.555552p-2f);
+    const float small = fmaf(a * z, p, a);
+    const float l2e2 = 0x1.715476p+1f, l2e2_lo = 0x1.4ae0c0p-25f;  // 2 log2(e)
+    const float h = a * l2e2;
+    const float lo = fmaf(a, l2e2_lo, fmaf(a, l2e2, -h));
+    const float e1 = __builtin_amdgcn_exp2f(h);
+    const float d = e1 + 1.0f;
+    const float dl = fmaf(e1, lo * 0x1.62e430p-1f, e1 - (d - 1.0f));  // e^(2a) + 1 = d + dl
+    float r = __builtin_amdgcn_rcpf(d);
+    r = fmaf(fmaf(-dl, r, fmaf(-d, r, 1.0f)), r, r);
+    const float big = a < 10.0f ? fmaf(-2.0f, r, 1.0f) : 1.0f;
+    return copysignf(a > 1.0f ? big : small, y);
+}
+template <bool VEC>
 __global__ void softcap_k(float* out, const float* in, float cap, int64_t n) {
-    AR_GRID_LOOP(i, n) out[i] = cap * tanhf(in[i] / cap);
+    if (VEC) {
+        AR_GRID_LOOP(i, n / 4) {
+            float4 x = reinterpret_cast<const float4*>(in)[i];
+            x.x = cap * tanh_pass(x.x / cap);
+            x.y = cap * tanh_pass(x.y / cap);
+            x.z = cap * tanh_pass(x.z / cap);
+            x.w = cap * tanh_pass(x.w / cap);
+            reinterpret_cast<float4*>(out)[i] = x;
+        }
+    } else {
+        AR_GRID_LOOP(i, n) out[i] = cap * tanh_pass(in[i] / cap);
+    }
 }
 
 // ---------------- K12 ve_apply_fwd ----------------
@@ -375,7 +417,10 @@ extern "C" int32_t ar_relu_squared_bwd(ar_stream_t stream, float* grad_input, co
 extern "C" int32_t ar_softcap_fwd(ar_stream_t stream, float* output, const float* input, float cap, int64_t size) {
     AR_ENSURE(output); AR_ENSURE(input); AR_NONNEG(size);
     if (size == 0) return AR_OK;
-    softcap_k<<<flat_grid(size, kBlock * 4), kBlock, 0, S(stream)>>>(output, input, cap, size);
+    if (size % 4 == 0 && al16(output) && al16(input))
+        softcap_k<true><<<grid_for<true>(size), kBlock, 0, S(stream)>>>(output, input, cap, size);
+    else
+        softcap_k<false><<<grid_for<false>(size), kBlock, 0, S(stream)>>>(output, input, cap, size);
     return AR_LAUNCH_CHECK("softcap_fwd");
 }
 

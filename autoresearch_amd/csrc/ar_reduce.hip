@@ -85,65 +85,136 @@ __global__ void rmsnorm_bwd_k(float* dx, const float* dy, const float* x, const 
     }
 }
 
-// Online (max, sum-exp) over one row by a block; every thread gets (m, s).
-__device__ __forceinline__ void row_max_sumexp(const float* row, int64_t n, float* red, float& m_out, float& s_out) {
-    float m = -INFINITY, s = 0.f;
-    for (int64_t i = threadIdx.x; i < n; i += blockDim.x) {
-        float v = row[i];
-        if (v > m) {
-            s = s * __expf(m - v) + 1.f;
-            m = v;
-        } else {
-            s += __expf(v - m);
-        }
-    }
-    const float bm = block_max(m, red);
-    s = (m == -INFINITY) ? 0.f : s * __expf(m - bm);
-    const float bs = block_sum(s, red + 32);
-    m_out = bm;
-    s_out = bs;
-}
+// ---------------- rows of exponentials: K15, K16, K18 ----------------
+// softmax_fwd (ops.mojo:600-666), cross_entropy_fwd (ops.mojo:672-740) and
+// cross_entropy_softcap_bwd (ops.mojo:778-864): one workgroup per row, HBM
+// bound (the row read once, for two of the three a row written).  A row of up
+// to 4 NV blockDim.x values is held in registers, 16 bytes per lane and load,
+// so that the maximum, the sum and the output come from one read and one
+// exponential per value; NV = 0 reads a longer row again for its output.
+// Rows are only 4-byte aligned (any V): the 16-byte accesses say so.
+// 8192 rows of 8192 (268 MB): loss 96 -> 49 us, gradient 180 -> 88 us
+// against one value per lane and load, two reads and two exponentials.
+typedef f32x4 f32x4u __attribute__((aligned(4)));
 
-// ---------------- K16 cross_entropy_fwd (ops.mojo:672-740) ----------------
-__global__ void ce_fwd_k(float* loss, const float* logits, const int64_t* targets, int64_t V) {
-    __shared__ float red[64];
-    const int64_t t = blockIdx.x;
-    const float* row = logits + t * V;
-    float m, s;
-    row_max_sumexp(row, V, red, m, s);
-    if (threadIdx.x == 0) {
-        const int64_t tg = targets[t];
-        const float lse = m + logf(s);
-        loss[t] = (tg >= 0 && tg < V) ? -row[tg] + lse : 0.f;  // out-of-range targets are ignored rows
-    }
+// Values 4c .. 4c + 3 of a row of n; -inf past its end (no weight).
+__device__ __forceinline__ f32x4 row_ld(const float* row, int64_t n, int64_t c) {
+    const int64_t i = 4 * c;
+    if (i + 4 <= n) return *reinterpret_cast<const f32x4u*>(row + i);
+    f32x4 x;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) x[e] = i + e < n ? row[i + e] : -INFINITY;
+    return x;
 }
-
-// ---------------- K18 cross_entropy_softcap_bwd (ops.mojo:778-864) ----------------
-__global__ void ce_bwd_k(float* grad, const float* logits, const int64_t* targets, int64_t V, float loss_scale) {
-    __shared__ float red[64];
-    const int64_t t = blockIdx.x;
-    const int64_t tg = targets[t];
-    float* g = grad + t * V;
-    if (tg < 0 || tg >= V) {
-        for (int64_t i = threadIdx.x; i < V; i += blockDim.x) g[i] = 0.f;
+__device__ __forceinline__ void row_st(float* row, int64_t n, int64_t c, f32x4 x) {
+    const int64_t i = 4 * c;
+    if (i + 4 <= n) {
+        *reinterpret_cast<f32x4u*>(row + i) = x;
         return;
     }
-    const float* row = logits + t * V;
-    float m, s;
-    row_max_sumexp(row, V, red, m, s);
-    for (int64_t i = threadIdx.x; i < V; i += blockDim.x) {
-        const float sm = __expf(row[i] - m) / s;
-        g[i] = (i == tg ? sm - 1.0f : sm) * loss_scale;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+        if (i + e < n) row[i + e] = x[e];
+}
+__device__ __forceinline__ float max4(f32x4 x) { return fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])); }
+__device__ __forceinline__ f32x4 exp4(f32x4 x, float m) {
+    f32x4 e;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) e[i] = __expf(x[i] - m);
+    return e;
+}
+// x / s (r = 1 / s): the quotient's remainder corrects it, as a division's would.
+__device__ __forceinline__ float div_by(float x, float s, float r) {
+    const float q = x * r;
+    return fmaf(fmaf(-q, s, x), r, q);
+}
+
+enum class RowOp { SOFTMAX, CE_FWD, CE_BWD };
+
+template <RowOp OP, int NV>
+__global__ __launch_bounds__(256) void exp_row_k(float* out, const float* in, const int64_t* targets, int64_t n,
+                                                 float loss_scale) {
+    __shared__ float red[64];
+    const int64_t r = blockIdx.x;
+    const float* row = in + r * n;
+    float* o = out + r * n;  // CE_FWD: unused
+    const int64_t nc = (n + 3) / 4;
+    int64_t tg = -1;
+    if constexpr (OP != RowOp::SOFTMAX) {
+        tg = targets[r];
+        if (tg < 0 || tg >= n) {  // out-of-range targets are ignored rows
+            if constexpr (OP == RowOp::CE_FWD) {
+                if (threadIdx.x == 0) out[r] = 0.f;
+            } else {
+                for (int64_t c = threadIdx.x; c < nc; c += blockDim.x) row_st(o, n, c, f32x4{0.f, 0.f, 0.f, 0.f});
+            }
+            return;
+        }
+    }
+    constexpr int NR = NV > 0 ? NV : 1;
+    f32x4 x[NR];
+    float m = -INFINITY, s = 0.f;
+    if constexpr (NV > 0) {
+#pragma unroll
+        for (int j = 0; j < NV; ++j) x[j] = row_ld(row, n, threadIdx.x + j * (int)blockDim.x);
+        float m4 = -INFINITY;
+#pragma unroll
+        for (int j = 0; j < NV; ++j) m4 = fmaxf(m4, max4(x[j]));
+        m = block_max(m4, red);
+#pragma unroll
+        for (int j = 0; j < NV; ++j) {
+            x[j] = exp4(x[j], m);
+            s += (x[j][0] + x[j][1]) + (x[j][2] + x[j][3]);
+        }
+    } else {
+        float mt = -INFINITY;
+        for (int64_t c = threadIdx.x; c < nc; c += blockDim.x) {
+            const f32x4 v = row_ld(row, n, c);
+            const float cm = max4(v);
+            if (cm > mt) {
+                s *= __expf(mt - cm);
+                mt = cm;
+            }
+            const f32x4 e = exp4(v, mt == -INFINITY ? 0.f : mt);
+            s += (e[0] + e[1]) + (e[2] + e[3]);
+        }
+        m = block_max(mt, red);
+        if (mt != -INFINITY) s *= __expf(mt - m);
+    }
+    s = block_sum(s, red + 32);
+    if constexpr (OP == RowOp::CE_FWD) {
+        if (threadIdx.x == 0) out[r] = -row[tg] + (m + logf(s));
+    } else {
+        const float rs = 1.0f / s;
+        auto emit = [&](int64_t c, f32x4 e) {
+            f32x4 y;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                y[i] = div_by(e[i], s, rs);
+                if constexpr (OP == RowOp::CE_BWD) y[i] = (4 * c + i == tg ? y[i] - 1.0f : y[i]) * loss_scale;
+            }
+            row_st(o, n, c, y);
+        };
+        if constexpr (NV > 0) {
+#pragma unroll
+            for (int j = 0; j < NV; ++j) emit(threadIdx.x + j * (int)blockDim.x, x[j]);
+        } else {
+            for (int64_t c = threadIdx.x; c < nc; c += blockDim.x) emit(c, exp4(row_ld(row, n, c), m));
+        }
     }
 }
 
-// ---------------- K15 softmax_fwd (ops.mojo:600-666) ----------------
-__global__ void softmax_k(float* out, const float* in, int64_t cols) {
-    __shared__ float red[64];
-    const int64_t r = blockIdx.x;
-    float m, s;
-    row_max_sumexp(in + r * cols, cols, red, m, s);
-    for (int64_t i = threadIdx.x; i < cols; i += blockDim.x) out[r * cols + i] = __expf(in[r * cols + i] - m) / s;
+// One wave holds a row of up to 2048 values (its reductions need no LDS trip
+// between waves), four waves up to 16384.
+template <RowOp OP>
+void exp_rows(hipStream_t st, float* out, const float* in, const int64_t* targets, int64_t rows, int64_t n,
+              float loss_scale) {
+    const unsigned g = (unsigned)rows;
+    if (n <= 512) exp_row_k<OP, 2><<<g, 64, 0, st>>>(out, in, targets, n, loss_scale);
+    else if (n <= 2048) exp_row_k<OP, 8><<<g, 64, 0, st>>>(out, in, targets, n, loss_scale);
+    else if (n <= 8192) exp_row_k<OP, 8><<<g, 256, 0, st>>>(out, in, targets, n, loss_scale);
+    else if (n <= 16384) exp_row_k<OP, 16><<<g, 256, 0, st>>>(out, in, targets, n, loss_scale);
+    else exp_row_k<OP, 0><<<g, 256, 0, st>>>(out, in, targets, n, loss_scale);
 }
 
 // ---------------- fixed-order multi-block sums ----------------
@@ -347,14 +418,20 @@ constexpr int kEmbChunk = 64;
 //   sort_scan_k     one workgroup turns hist into exclusive offsets in that
 //                   order (all of digit 0 over the tiles in order, then digit
 //                   1, ...), i.e. the first output slot of (digit, tile);
-//   sort_scatter_k  one wave per tile walks its positions in order, 64 at a
-//                   time: the lanes holding the same digit are found with one
-//                   ballot per digit bit, ranked by lane, and placed after the
-//                   (digit, tile) offset advanced by the earlier rounds.
-// Tiles, rounds and lanes are visited in position order, so equal digits keep
-// their input order (stable), and the result is the same on every run.
+//   sort_scatter_k  a tile's 16 waves take 128 consecutive positions each, 64
+//                   at a time: the lanes holding the same digit are found with
+//                   one ballot per digit bit and ranked by lane after the
+//                   wave's earlier round; the waves' counts per digit, summed
+//                   in wave order, place each after the (digit, tile) offset.
+//                   What bounds it is the chain of rounds: with one wave per
+//                   tile walking all 32 (8192 ids, 11 bits) 35 us a pass,
+//                   7 us with 16.
+// Tiles, waves, rounds and lanes are ranked in position order, so equal digits
+// keep their input order (stable), and the result is the same on every run.
 constexpr int kSortTile = 2048;
 constexpr int kSortMaxBits = 11;
+constexpr int kSortWaves = 16, kSortThreads = kSortWaves * kWave;
+constexpr int kSortRounds = kSortTile / kSortThreads;
 
 __global__ __launch_bounds__(256) void sort_hist_k(int32_t* hist, const int64_t* ids, const uint32_t* keys, int64_t n,
                                                     int shift, int bits, int64_t ntiles) {
@@ -400,27 +477,39 @@ __global__ __launch_bounds__(1024) void sort_scan_k(int32_t* v, int64_t total) {
     }
 }
 
-__global__ __launch_bounds__(64) void sort_scatter_k(uint32_t* keys_out, int32_t* vals_out, const int64_t* ids,
-                                                     const uint32_t* keys_in, const int32_t* vals_in,
-                                                     const int32_t* hist, int64_t n, int shift, int bits,
-                                                     int64_t ntiles) {
+__global__ __launch_bounds__(kSortThreads) void sort_scatter_k(uint32_t* keys_out, int32_t* vals_out,
+                                                               const int64_t* ids, const uint32_t* keys_in,
+                                                               const int32_t* vals_in, const int32_t* hist, int64_t n,
+                                                               int shift, int bits, int64_t ntiles) {
+    __shared__ uint16_t cnt[kSortWaves][1 << kSortMaxBits];  // per wave: its count, then the slots taken before it
     __shared__ int32_t base[1 << kSortMaxBits];
-    const int lane = threadIdx.x;
+    const int lane = threadIdx.x % kWave, w = threadIdx.x / kWave;
     const int bins = 1 << bits;
-    for (int d = lane; d < bins; d += 64) base[d] = hist[(int64_t)d * ntiles + blockIdx.x];
-    __syncthreads();
-    const int64_t t0 = (int64_t)blockIdx.x * kSortTile;
-    const uint64_t below = lane == 0 ? 0ull : (~0ull >> (64 - lane));
-    for (int r = 0; r < kSortTile && t0 + r < n; r += 64) {  // wave-uniform bounds
-        const int64_t p = t0 + r + lane;
-        const bool valid = p < n;
-        uint32_t k = 0;
-        int32_t v = 0;
-        if (valid) {
-            k = ids ? (uint32_t)ids[p] : keys_in[p];
-            v = ids ? (int32_t)p : vals_in[p];
+    for (int d = threadIdx.x; d < bins; d += kSortThreads) {
+        base[d] = hist[(int64_t)d * ntiles + blockIdx.x];
+#pragma unroll
+        for (int u = 0; u < kSortWaves; ++u) cnt[u][d] = 0;
+    }
+    const int64_t p0 = (int64_t)blockIdx.x * kSortTile + w * (kSortRounds * kWave) + lane;
+    uint32_t k[kSortRounds];
+    int32_t v[kSortRounds];
+    int rank[kSortRounds];  // among the wave's own positions of the same digit
+#pragma unroll
+    for (int r = 0; r < kSortRounds; ++r) {
+        const int64_t p = p0 + r * kWave;
+        k[r] = 0;
+        v[r] = 0;
+        if (p < n) {
+            k[r] = ids ? (uint32_t)ids[p] : keys_in[p];
+            v[r] = ids ? (int32_t)p : vals_in[p];
         }
-        const uint32_t d = (k >> shift) & (uint32_t)(bins - 1);
+    }
+    __syncthreads();
+    const uint64_t below = lane == 0 ? 0ull : (~0ull >> (64 - lane));
+#pragma unroll
+    for (int r = 0; r < kSortRounds; ++r) {
+        const bool valid = p0 + r * kWave < n;
+        const uint32_t d = (k[r] >> shift) & (uint32_t)(bins - 1);
         uint64_t peers = __ballot(valid);
         for (int bit = 0; bit < bits; ++bit) {
             const bool on = (d >> bit) & 1u;
@@ -428,16 +517,29 @@ __global__ __launch_bounds__(64) void sort_scatter_k(uint32_t* keys_out, int32_t
             peers &= on ? bal : ~bal;
         }
         // peers: the valid lanes holding digit d (this lane included when valid)
-        const int leader = valid ? __ffsll((unsigned long long)peers) - 1 : lane;
-        int32_t b0 = (valid && lane == leader) ? base[d] : 0;
-        b0 = __shfl(b0, leader, 64);
-        if (valid) {
-            const int32_t pos = b0 + __popcll(peers & below);
-            keys_out[pos] = k;
-            vals_out[pos] = v;
-            if (lane == leader) base[d] = b0 + __popcll(peers);
+        const int before = valid ? cnt[w][d] : 0;
+        rank[r] = before + __popcll(peers & below);
+        __syncthreads();  // every lane has read its count before its digit's first lane advances it
+        if (valid && (peers & below) == 0) cnt[w][d] = (uint16_t)(before + __popcll(peers));
+        __syncthreads();
+    }
+    for (int d = threadIdx.x; d < bins; d += kSortThreads) {
+        int run = 0;
+#pragma unroll
+        for (int u = 0; u < kSortWaves; ++u) {
+            const int c = cnt[u][d];
+            cnt[u][d] = (uint16_t)run;
+            run += c;
         }
-        __syncthreads();  // the next round's leaders read the advanced offsets
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kSortRounds; ++r) {
+        if (p0 + r * kWave >= n) continue;
+        const uint32_t d = (k[r] >> shift) & (uint32_t)(bins - 1);
+        const int32_t pos = base[d] + cnt[w][d] + rank[r];
+        keys_out[pos] = k[r];
+        vals_out[pos] = v[r];
     }
 }
 
@@ -661,7 +763,7 @@ extern "C" int32_t ar_cross_entropy_fwd(ar_stream_t stream, float* loss_out, con
     AR_CHECK_ARG(loss_out && logits && targets, "cross_entropy_fwd: null pointer");
     AR_CHECK_ARG(num_tokens >= 0 && vocab_size > 0, "cross_entropy_fwd: bad shape");
     if (num_tokens == 0) return AR_OK;
-    ce_fwd_k<<<(unsigned)num_tokens, kBlock, 0, S(stream)>>>(loss_out, logits, targets, vocab_size);
+    exp_rows<RowOp::CE_FWD>(S(stream), loss_out, logits, targets, num_tokens, vocab_size, 1.0f);
     return AR_LAUNCH_CHECK("cross_entropy_fwd");
 }
 
@@ -672,7 +774,7 @@ extern "C" int32_t ar_cross_entropy_softcap_bwd(ar_stream_t stream, float* grad_
     AR_CHECK_ARG(grad_logits && logits && targets, "cross_entropy_softcap_bwd: null pointer");
     AR_CHECK_ARG(num_tokens >= 0 && vocab_size > 0, "cross_entropy_softcap_bwd: bad shape");
     if (num_tokens == 0) return AR_OK;
-    ce_bwd_k<<<(unsigned)num_tokens, kBlock, 0, S(stream)>>>(grad_logits, logits, targets, vocab_size, loss_scale);
+    exp_rows<RowOp::CE_BWD>(S(stream), grad_logits, logits, targets, num_tokens, vocab_size, loss_scale);
     return AR_LAUNCH_CHECK("cross_entropy_softcap_bwd");
 }
 
@@ -681,7 +783,7 @@ extern "C" int32_t ar_softmax_fwd(ar_stream_t stream, float* output, const float
     AR_CHECK_ARG(output && input, "softmax_fwd: null pointer");
     AR_CHECK_ARG(num_rows >= 0 && cols > 0, "softmax_fwd: bad shape");
     if (num_rows == 0) return AR_OK;
-    softmax_k<<<(unsigned)num_rows, kBlock, 0, S(stream)>>>(output, input, cols);
+    exp_rows<RowOp::SOFTMAX>(S(stream), output, input, nullptr, num_rows, cols, 1.0f);
     return AR_LAUNCH_CHECK("softmax_fwd");
 }
 
@@ -884,7 +986,7 @@ extern "C" int32_t ar_embedding_sort(ar_stream_t stream, uint32_t* sorted_ids, i
         const int64_t* ids = p == 0 ? indices : nullptr;
         sort_hist_k<<<(unsigned)ntiles, 256, 0, st>>>(hist, ids, kin, n, shift, pb, ntiles);
         sort_scan_k<<<1, 1024, 0, st>>>(hist, (int64_t)(1 << pb) * ntiles);
-        sort_scatter_k<<<(unsigned)ntiles, 64, 0, st>>>(kout, vout, ids, kin, vin, hist, n, shift, pb, ntiles);
+        sort_scatter_k<<<(unsigned)ntiles, kSortThreads, 0, st>>>(kout, vout, ids, kin, vin, hist, n, shift, pb, ntiles);
         kin = kout;
         vin = vout;
     }
