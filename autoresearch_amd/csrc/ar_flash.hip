@@ -204,6 +204,31 @@ __device__ __forceinline__ void dma_tile(bf16* dst, const bf16* base, int64_t rs
     }
 }
 
+// ---- own rows in fp32 ----
+// The calls whose tensors are fp32 (any head_dim hd <= HD) stream rounded,
+// zero-padded copies, which several workgroups read, but a workgroup's own
+// rows, read once, come straight from the fp32 tensor and are rounded on the
+// way, and results go straight to the hd columns of the fp32 output.
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+
+// Eight values rounded to bf16, the first n of them from p, the others zero
+// (rows are 4-byte aligned when hd is not a multiple of 4).
+__device__ __forceinline__ bf16x8 ld8_bf16(const float* p, int n) {
+    bf16x8 f;
+    if (n >= 8) {
+        const f32x4u a = *reinterpret_cast<const f32x4u*>(p), b = *reinterpret_cast<const f32x4u*>(p + 4);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            f[e] = (bf16)a[e];
+            f[4 + e] = (bf16)b[e];
+        }
+    } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) f[e] = e < n ? (bf16)p[e] : (bf16)0.0f;
+    }
+    return f;
+}
+
 // B fragments of 32 own rows (row = row0 + lane % 32), read from global.
 template <int HD>
 __device__ __forceinline__ void own_frags(bf16x8 (&f)[HD / 16], const bf16* base, int64_t rs, int row, int T,
@@ -216,6 +241,35 @@ __device__ __forceinline__ void own_frags(bf16x8 (&f)[HD / 16], const bf16* base
 #pragma unroll
             for (int e = 0; e < 8; ++e) f[ks][e] = (bf16)0.0f;
         }
+    }
+}
+
+template <int HD>
+__device__ __forceinline__ void own_frags(bf16x8 (&f)[HD / 16], const float* base, int64_t rs, int row, int T,
+                                          int lane, int hd) {
+#pragma unroll
+    for (int ks = 0; ks < HD / 16; ++ks) {
+        const int c = ks * 16 + (lane >> 5) * 8;
+        f[ks] = ld8_bf16(base + (int64_t)row * rs + c, row < T ? hd - c : 0);
+    }
+}
+template <int HD>
+__device__ __forceinline__ void own_frags(bf16x8 (&f)[HD / 16], const bf16* base, int64_t rs, int row, int T,
+                                          int lane, int) {
+    own_frags<HD>(f, base, rs, row, T, lane);
+}
+
+// The kOwn own rows in the swizzled natural layout, rounded from fp32 (rows
+// past T repeat row T - 1, as dma_tile's do).
+template <int HD>
+__device__ __forceinline__ void own_tile(bf16* dst, const float* base, int64_t rs, int row0, int T, int hd) {
+    using G = Geo<HD>;
+#pragma unroll 4
+    for (int i = 0; i < TileU<HD, kOwn>::N; ++i) {
+        const int id = i * kThreads + threadIdx.x;
+        const int r = id / G::NCH, c = ((id % G::NCH) ^ G::swz(r)) * 8;
+        const int row = row0 + r < T ? row0 + r : T - 1;
+        *reinterpret_cast<bf16x8*>(dst + id * 8) = ld8_bf16(base + (int64_t)row * rs + c, hd - c);
     }
 }
 
@@ -259,9 +313,21 @@ __device__ __forceinline__ void st_nt(bf16* p, bf16x4 v) {
     __builtin_nontemporal_store(__builtin_bit_cast(unsigned long long, v), reinterpret_cast<unsigned long long*>(p));
 }
 
-template <int HD>
+// st_nt of the columns d .. d + 3 that are below hd.
+__device__ __forceinline__ void st_nt_below(float* p, float4 x, int d, int hd) {
+    if (d + 4 <= hd) {
+        st_nt(p, x);
+        return;
+    }
+    if (d < hd) __builtin_nontemporal_store(x.x, p);
+    if (d + 1 < hd) __builtin_nontemporal_store(x.y, p + 1);
+    if (d + 2 < hd) __builtin_nontemporal_store(x.z, p + 2);
+}
+
+// With F32 the rows are fp32 and hd <= HD columns wide.
+template <int HD, bool F32>
 __device__ __forceinline__ void store_rows(const RowOut& o, int row_base, int T, const f32x16 (&acc)[HD / 32],
-                                           float colscale, float* scratch, int lane) {
+                                           float colscale, float* scratch, int lane, int hd) {
     constexpr int DT = HD / 32, HALF = HD / 2;
     constexpr int NPAIR = DT >= 2 ? DT / 2 : 1;  // staged (block, block + DT/2) pairs
     constexpr int PW = DT >= 2 ? 32 : 16;        // pair columns per staged block
@@ -284,6 +350,11 @@ __device__ __forceinline__ void store_rows(const RowOut& o, int row_base, int T,
             float4 x1 = *reinterpret_cast<const float4*>(scratch + r * LDS_ + c4);
             float4 x2 = *reinterpret_cast<const float4*>(scratch + r * LDS_ + (DT >= 2 ? 32 : 16) + c4);
             const int d1 = (DT >= 2 ? p * 32 : 0) + c4, d2 = d1 + HALF;
+            if constexpr (F32) {
+                st_nt_below(o.of + (int64_t)row * o.rsf + d1, x1, d1, hd);
+                st_nt_below(o.of + (int64_t)row * o.rsf + d2, x2, d2, hd);
+                continue;
+            }
             if (o.of) {
                 st_nt(o.of + (int64_t)row * o.rsf + d1, x1);
                 st_nt(o.of + (int64_t)row * o.rsf + d2, x2);
@@ -329,10 +400,11 @@ __device__ __forceinline__ bool visible(int kp, int qp, int T, int window) {
 
 // ============================ forward ============================
 // Two workgroups per CU (2 waves per SIMD): registers are capped at 256.
-template <int HD>
-__global__ __launch_bounds__(kThreads, 2) void fa2_fwd_k(RowOut out, float* lse, const bf16* q, const bf16* k,
+template <int HD, typename OWN>
+__global__ __launch_bounds__(kThreads, 2) void fa2_fwd_k(RowOut out, float* lse, const OWN* q, const bf16* k,
                                                          const bf16* v, int B, int T, int H, int window,
-                                                         float scale_log2) {
+                                                         float scale_log2, int hd) {
+    constexpr bool F32 = std::is_same<OWN, float>::value;
     using G = Geo<HD>;
     extern __shared__ __align__(16) unsigned char smem_raw[];
     bf16* const lds = reinterpret_cast<bf16*>(smem_raw);  // stage s: K at 2 s TILE, V at (2 s + 1) TILE
@@ -345,8 +417,10 @@ __global__ __launch_bounds__(kThreads, 2) void fa2_fwd_k(RowOut out, float* lse,
     const int64_t rs = (int64_t)H * HD;
     const int64_t boff = (int64_t)b * T * rs + (int64_t)h * HD;
 
+    const int ohd = F32 ? hd : HD;  // columns of an own row
+    const int64_t ors = (int64_t)H * ohd, ooff = (int64_t)b * T * ors + (int64_t)h * ohd;
     bf16x8 qf[G::KSTEPS];
-    own_frags<HD>(qf, q + boff, rs, my_q, T, lane);
+    own_frags<HD>(qf, q + ooff, ors, my_q, T, lane, hd);
     f32x16 o[G::DT];
 #pragma unroll
     for (int dt = 0; dt < G::DT; ++dt)
@@ -509,15 +583,16 @@ __global__ __launch_bounds__(kThreads, 2) void fa2_fwd_k(RowOut out, float* lse,
     const float inv_l = l > 0.f ? 1.0f / l : 0.f;
     if (lane < 32 && my_q < T) lse[((int64_t)b * T + my_q) * H + h] = l > 0.f ? (m + log2f(l)) * kLn2 : -INFINITY;
     float* scratch = reinterpret_cast<float*>(smem_raw) + wave * 32 * 68;
-    store_rows<HD>(at_head(out, b, h, T, HD), qw, T, o, inv_l, scratch, lane);
+    store_rows<HD, F32>(at_head(out, b, h, T, ohd), qw, T, o, inv_l, scratch, lane, hd);
 }
 
 // ============================ backward: dQ ============================
-template <int HD>
-__global__ __launch_bounds__(kThreads, 2) void fa2_dq_k(RowOut dq, const bf16* q, const bf16* k, const bf16* v,
-                                                     const bf16* dout, const float* lse, const float* dbuf,
+template <int HD, typename OWN>
+__global__ __launch_bounds__(kThreads, 2) void fa2_dq_k(RowOut dq, const OWN* q, const bf16* k, const bf16* v,
+                                                     const OWN* dout, const float* lse, const float* dbuf,
                                                      int B, int T, int H, int window, float scale_log2,
-                                                     float scale) {
+                                                     float scale, int hd) {
+    constexpr bool F32 = std::is_same<OWN, float>::value;
     using G = Geo<HD>;
     extern __shared__ __align__(16) unsigned char smem_raw[];
     bf16* const lds = reinterpret_cast<bf16*>(smem_raw);  // stage s: K at 2 s TILE, V at (2 s + 1) TILE
@@ -530,9 +605,11 @@ __global__ __launch_bounds__(kThreads, 2) void fa2_dq_k(RowOut dq, const bf16* q
     const int64_t rs = (int64_t)H * HD;
     const int64_t boff = (int64_t)b * T * rs + (int64_t)h * HD;
 
+    const int ohd = F32 ? hd : HD;  // columns of an own row
+    const int64_t ors = (int64_t)H * ohd, ooff = (int64_t)b * T * ors + (int64_t)h * ohd;
     bf16x8 qf[G::KSTEPS], df[G::KSTEPS];
-    own_frags<HD>(qf, q + boff, rs, my_q, T, lane);
-    own_frags<HD>(df, dout + boff, rs, my_q, T, lane);
+    own_frags<HD>(qf, q + ooff, ors, my_q, T, lane, hd);
+    own_frags<HD>(df, dout + ooff, ors, my_q, T, lane, hd);
     const int64_t bth = ((int64_t)b * T + (my_q < T ? my_q : 0)) * H + h;
     const float my_lse2 = lse[bth] * kLog2e;
     const float my_D = dbuf[bth];
@@ -612,7 +689,7 @@ __global__ __launch_bounds__(kThreads, 2) void fa2_dq_k(RowOut dq, const bf16* q
         __syncthreads();
     }
     float* scratch = reinterpret_cast<float*>(smem_raw) + wave * 32 * 68;
-    store_rows<HD>(at_head(dq, b, h, T, HD), qw, T, acc, scale, scratch, lane);
+    store_rows<HD, F32>(at_head(dq, b, h, T, ohd), qw, T, acc, scale, scratch, lane, hd);
 }
 
 // ============================ backward: dK, dV ============================
@@ -672,12 +749,13 @@ constexpr size_t dkv_fused_lds() {
     return loop > stage ? loop : stage;
 }
 
-template <int HD, bool WDS>
+template <int HD, bool WDS, typename OWN>
 __global__ __launch_bounds__(kThreads, 2) void fa2_dkv_fused_k(RowOut out_k, RowOut out_v, const bf16* q,
-                                                               const bf16* k, const bf16* v, const bf16* dout,
+                                                               const OWN* k, const OWN* v, const bf16* dout,
                                                                const float* lse, const float* dbuf, bf16* ds_out,
                                                                int B, int T, int H, int window, float scale_log2,
-                                                               float scale) {
+                                                               float scale, int hd) {
+    constexpr bool F32 = std::is_same<OWN, float>::value;
     using G = Geo<HD>;
     constexpr int KT = kDkvTile, TT = KT * HD;  // rows, bf16 elements per streamed tile
     extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -694,8 +772,10 @@ __global__ __launch_bounds__(kThreads, 2) void fa2_dkv_fused_k(RowOut out_k, Row
     const int64_t rs = (int64_t)H * HD;
     const int64_t boff = (int64_t)b * T * rs + (int64_t)h * HD;
 
+    const int ohd = F32 ? hd : HD;  // columns of an own row
+    const int64_t ors = (int64_t)H * ohd, ooff = (int64_t)b * T * ors + (int64_t)h * ohd;
     bf16x8 kf[G::KSTEPS];
-    own_frags<HD>(kf, k + boff, rs, my_k, T, lane);
+    own_frags<HD>(kf, k + ooff, ors, my_k, T, lane, hd);
 
     f32x16 adk[G::DT], adv[G::DT];
 #pragma unroll
@@ -718,7 +798,9 @@ __global__ __launch_bounds__(kThreads, 2) void fa2_dkv_fused_k(RowOut out_k, Row
             dma4(lane < KT ? lse + i : dbuf + i, lds_addr(sLD + stage * 2 * KT));
         }
     };
-    {
+    if constexpr (F32) {
+        own_tile<HD>(sV, v + ooff, ors, k0, T, hd);
+    } else {
         unsigned voff[TileU<HD, kOwn>::N];
         tile_offsets<HD, kOwn>(voff, rs);
         dma_tile<HD, kOwn>(sV, v + boff, rs, k0, T, voff);
@@ -827,8 +909,8 @@ __global__ __launch_bounds__(kThreads, 2) void fa2_dkv_fused_k(RowOut out_k, Row
         __syncthreads();
     }
     float* scratch = reinterpret_cast<float*>(smem_raw) + wave * 32 * 68;
-    store_rows<HD>(at_head(out_v, b, h, T, HD), kw, T, adv, 1.0f, scratch, lane);
-    store_rows<HD>(at_head(out_k, b, h, T, HD), kw, T, adk, scale, scratch, lane);
+    store_rows<HD, F32>(at_head(out_v, b, h, T, ohd), kw, T, adv, 1.0f, scratch, lane, hd);
+    store_rows<HD, F32>(at_head(out_k, b, h, T, ohd), kw, T, adk, scale, scratch, lane, hd);
 }
 
 // ============================ backward: dQ from stored dS ============================
@@ -948,7 +1030,7 @@ __global__ __launch_bounds__(kDqThreads) void fa2_dq_ds_k(RowOut dq, const bf16*
         __syncthreads();
     }
     float* scratch = reinterpret_cast<float*>(smem_raw) + wave * 32 * 68;
-    store_rows<HD>(at_head(dq, b, h, T, HD), qw, T, acc, scale, scratch, lane);
+    store_rows<HD, false>(at_head(dq, b, h, T, HD), qw, T, acc, scale, scratch, lane, HD);
 }
 
 // D = rowsum(dO * O) (ops.mojo:329-346) per (token, head) row: bf16 dO (the
@@ -988,32 +1070,75 @@ constexpr size_t fa2_lds(bool with_ld) {
 template <int HD>
 int32_t flash_hd(hipStream_t st, AttnOp op, float* o1, float* o2, const FlashOut& fo, const bf16* q, const bf16* k,
                  const bf16* v, const bf16* dout, const float* lse, const float* dbuf, int B, int T, int H,
-                 int window, float sc) {
-    const float scale = sc > 0.f ? sc : 1.0f / sqrtf((float)HD);
+                 int window) {
+    const float scale = 1.0f / sqrtf((float)HD);
     const float scale_log2 = scale * kLog2e;
     const unsigned grid = (unsigned)(((T + kOwn - 1) / kOwn) * B * H);
     const int64_t rs = (int64_t)H * HD, brs = fo.brs > 0 ? fo.brs : rs;
     if (op == AttnOp::FWD) {
         const RowOut out{o1, fo.b1, rs, brs, nullptr, nullptr, 0, 1};
-        fa2_fwd_k<HD><<<grid, kThreads, fa2_lds<HD>(false), st>>>(out, o2, q, k, v, B, T, H, window, scale_log2);
+        fa2_fwd_k<HD, bf16><<<grid, kThreads, fa2_lds<HD>(false), st>>>(out, o2, q, k, v, B, T, H, window, scale_log2,
+                                                                        HD);
         return check_launch("flash_attn_fwd (bf16 operands)");
     }
     const int64_t period = fo.period > 0 ? fo.period : (int64_t)B * T;
     if (op == AttnOp::DQ) {
         const RowOut out{o1, fo.b1, rs, brs, fo.cos_t, fo.sin_t, 0, period};
-        fa2_dq_k<HD><<<grid, kThreads, fa2_lds<HD>(false), st>>>(out, q, k, v, dout, lse, dbuf, B, T, H, window,
-                                                                 scale_log2, scale);
+        fa2_dq_k<HD, bf16><<<grid, kThreads, fa2_lds<HD>(false), st>>>(out, q, k, v, dout, lse, dbuf, B, T, H, window,
+                                                                       scale_log2, scale, HD);
         return check_launch("flash_attn_bwd_dq (bf16 operands)");
     }
     const RowOut ov{o2, fo.b2, rs, brs, nullptr, nullptr, 0, 1};
     const RowOut ok{o1, fo.b1, rs, brs, fo.cos_t, fo.sin_t, 0, period};
     if (fo.ds)
-        fa2_dkv_fused_k<HD, true><<<grid, kThreads, dkv_fused_lds<HD, true>(), st>>>(ok, ov, q, k, v, dout, lse, dbuf, fo.ds,
-                                                                          B, T, H, window, scale_log2, scale);
+        fa2_dkv_fused_k<HD, true, bf16><<<grid, kThreads, dkv_fused_lds<HD, true>(), st>>>(
+            ok, ov, q, k, v, dout, lse, dbuf, fo.ds, B, T, H, window, scale_log2, scale, HD);
     else
-        fa2_dkv_fused_k<HD, false><<<grid, kThreads, dkv_fused_lds<HD, false>(), st>>>(ok, ov, q, k, v, dout, lse, dbuf,
-                                                                           nullptr, B, T, H, window, scale_log2, scale);
+        fa2_dkv_fused_k<HD, false, bf16><<<grid, kThreads, dkv_fused_lds<HD, false>(), st>>>(
+            ok, ov, q, k, v, dout, lse, dbuf, nullptr, B, T, H, window, scale_log2, scale, HD);
     return check_launch("flash_attn_bwd_dkv (bf16 operands)");
+}
+
+// The streamed pair of an op on fp32 tensors: rows rounded to bf16 and
+// zero-padded from hd to HD columns, both tensors in one launch (blockIdx.y),
+// eight columns per thread.
+template <int HD>
+__global__ __launch_bounds__(kThreads) void round_rows_k(bf16* d0, bf16* d1, const float* s0, const float* s1,
+                                                         int64_t rows, int hd) {
+    constexpr int CH = HD / 8;
+    bf16* const dst = blockIdx.y ? d1 : d0;
+    const float* const src = blockIdx.y ? s1 : s0;
+    for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < rows * CH; i += (int64_t)gridDim.x * kThreads) {
+        const int64_t r = i / CH;
+        const int c = (int)(i % CH) * 8;
+        *reinterpret_cast<bf16x8*>(dst + i * 8) = ld8_bf16(src + r * hd + c, hd - c);
+    }
+}
+
+template <int HD>
+int32_t flash_f32_hd(hipStream_t st, AttnOp op, float* o1, float* o2, const float* q, const float* k, const float* v,
+                     const float* dout, const float* lse, const float* dbuf, int B, int T, int H, int hd, int window,
+                     bf16* w0, bf16* w1) {
+    const float scale = 1.0f / sqrtf((float)hd);
+    const float scale_log2 = scale * kLog2e;
+    const unsigned grid = (unsigned)(((T + kOwn - 1) / kOwn) * B * H);
+    const int64_t rs = (int64_t)H * hd, rows = (int64_t)B * T * H;
+    const RowOut out1{o1, nullptr, rs, rs, nullptr, nullptr, 0, 1}, out2{o2, nullptr, rs, rs, nullptr, nullptr, 0, 1};
+    const dim3 rgrid(flat_grid(rows * (HD / 8), kThreads), 2);
+    if (op == AttnOp::DKV)
+        round_rows_k<HD><<<rgrid, kThreads, 0, st>>>(w0, w1, q, dout, rows, hd);
+    else
+        round_rows_k<HD><<<rgrid, kThreads, 0, st>>>(w0, w1, k, v, rows, hd);
+    if (op == AttnOp::FWD)
+        fa2_fwd_k<HD, float><<<grid, kThreads, fa2_lds<HD>(false), st>>>(out1, o2, q, w0, w1, B, T, H, window,
+                                                                         scale_log2, hd);
+    else if (op == AttnOp::DQ)
+        fa2_dq_k<HD, float><<<grid, kThreads, fa2_lds<HD>(false), st>>>(out1, q, w0, w1, dout, lse, dbuf, B, T, H,
+                                                                        window, scale_log2, scale, hd);
+    else
+        fa2_dkv_fused_k<HD, false, float><<<grid, kThreads, dkv_fused_lds<HD, false>(), st>>>(
+            out1, out2, w0, k, v, w1, lse, dbuf, nullptr, B, T, H, window, scale_log2, scale, hd);
+    return check_launch("flash attention (bf16 products of fp32 tensors)");
 }
 
 template <int HD>
@@ -1065,17 +1190,29 @@ int32_t flash_dq_ds_bf16(hipStream_t st, const FlashOut& fo, const bf16* k, cons
 
 int32_t flash_attn_bf16(hipStream_t st, AttnOp op, float* o1, float* o2, const FlashOut& fo, const bf16* q,
                         const bf16* k, const bf16* v, const bf16* dout, const float* lse, const float* dbuf, int64_t B,
-                        int64_t T, int64_t H, int64_t HD, int64_t window, float scale) {
+                        int64_t T, int64_t H, int64_t HD, int64_t window) {
     if (B <= 0 || T <= 0 || H <= 0) return B == 0 || T == 0 ? AR_OK : set_error(AR_EINVAL, "flash attention: bad shape");
     if (((T + kOwn - 1) / kOwn) * B * H > 0x7fffffff || T > (1 << 30))
         return set_error(AR_EINVAL, "flash attention: shape too large");
     const int w = window > T ? (int)T : (int)window;  // a window >= T is full causal
     switch (HD) {
-        case 32: return flash_hd<32>(st, op, o1, o2, fo, q, k, v, dout, lse, dbuf, (int)B, (int)T, (int)H, w, scale);
-        case 64: return flash_hd<64>(st, op, o1, o2, fo, q, k, v, dout, lse, dbuf, (int)B, (int)T, (int)H, w, scale);
-        case 128: return flash_hd<128>(st, op, o1, o2, fo, q, k, v, dout, lse, dbuf, (int)B, (int)T, (int)H, w, scale);
+        case 32: return flash_hd<32>(st, op, o1, o2, fo, q, k, v, dout, lse, dbuf, (int)B, (int)T, (int)H, w);
+        case 64: return flash_hd<64>(st, op, o1, o2, fo, q, k, v, dout, lse, dbuf, (int)B, (int)T, (int)H, w);
+        case 128: return flash_hd<128>(st, op, o1, o2, fo, q, k, v, dout, lse, dbuf, (int)B, (int)T, (int)H, w);
         default: return set_error(AR_EUNSUPPORTED, "flash attention: head_dim %lld not in {32, 64, 128}", (long long)HD);
     }
+}
+
+int32_t flash_attn_f32(hipStream_t st, AttnOp op, float* o1, float* o2, const float* q, const float* k,
+                       const float* v, const float* dout, const float* lse, const float* dbuf, int64_t B, int64_t T,
+                       int64_t H, int64_t hd, int64_t window, bf16* w0, bf16* w1) {
+    if (((T + kOwn - 1) / kOwn) * B * H > 0x7fffffff || T > (1 << 30))
+        return set_error(AR_EINVAL, "flash attention: shape too large");
+    const int w = window > T ? (int)T : (int)window;
+    const int b = (int)B, t = (int)T, h = (int)H, d = (int)hd;
+    if (hd <= 32) return flash_f32_hd<32>(st, op, o1, o2, q, k, v, dout, lse, dbuf, b, t, h, d, w, w0, w1);
+    if (hd <= 64) return flash_f32_hd<64>(st, op, o1, o2, q, k, v, dout, lse, dbuf, b, t, h, d, w, w0, w1);
+    return flash_f32_hd<128>(st, op, o1, o2, q, k, v, dout, lse, dbuf, b, t, h, d, w, w0, w1);
 }
 
 }  // namespace ar
