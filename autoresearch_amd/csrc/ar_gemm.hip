@@ -474,7 +474,8 @@ __global__ void splitk_reduce_k(TC* C, const float* partial, int64_t M, int64_t 
 // lane fetches: a per-lane 32-bit offset fixed for the whole kernel, added to
 // a wave-uniform (SGPR) base that moves by one k-tile per copy and is set
 // once per tile, so a copy costs a few scalar instructions.  The epilogue stages 16-row half strips (fp32) in a separate
-// 32 KB region.  Shapes: M, N % 256, K (per split) % 64, lda/ldb % 8.
+// 32 KB region.  Shapes: M, N % 8 (whole or edge tiles), K (per split) % 64,
+// lda/ldb % 8.
 constexpr int kPkThreads = 512, kPkBK = 64, kPkStage = 2 * 256 * kPkBK * 2;  // bytes per stage (A + B)
 constexpr int kPkLds = 2 * kPkStage + 8 * 16 * 64 * 4;                      // 160 KB
 
@@ -488,18 +489,20 @@ __device__ __forceinline__ void vm_wait() {
 // Per-lane byte offsets of the 4 DMA wave-instructions that fill one operand
 // tile, relative to the tile's first element (row0, k0): slot (8j + w)*64 +
 // lane of wave w, swizzled as the tile layout above says.  Constant for the
-// whole kernel; the tile position goes into a wave-uniform base address.
+// whole kernel (with whole tiles); the tile position goes into a wave-uniform
+// base address.  Of an edge tile only the first `lim` rows (a multiple of 8)
+// exist: the others repeat the last row or 8-row unit.
 template <bool KMAJ>
-__device__ __forceinline__ void pk_offsets(unsigned (&off)[4], int ld, int wave, int lane) {
+__device__ __forceinline__ void pk_offsets(unsigned (&off)[4], int ld, int wave, int lane, int lim = 256) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         const int slot = (j * 8 + wave) * 64 + lane;
         if constexpr (KMAJ) {
             const int r = slot >> 3, c = (slot & 7) ^ ((r >> 1) & 7);
-            off[j] = (unsigned)(r * ld + c * 8) * 2u;
+            off[j] = (unsigned)((r < lim ? r : lim - 1) * ld + c * 8) * 2u;
         } else {
             const int k = slot >> 5, c = (slot & 31) ^ tr_swz(k);
-            off[j] = (unsigned)(k * ld + c * 8) * 2u;
+            off[j] = (unsigned)(k * ld + (c * 8 < lim ? c * 8 : lim - 8)) * 2u;
         }
     }
 }
@@ -532,8 +535,9 @@ struct PkHead {
 
 // HLD = 0: 8 waves of 128 x 64.  HLD = head_dim (32 / 64 / 128): 8 waves of
 // 64 x 128 (4 x 2), so each wave's 128 output columns hold whole heads, for
-// the head-wise epilogues.
-template <bool AK, bool BKM, typename TC, int EPI, int HLD = 0>
+// the head-wise epilogues.  EDGE: M or N is a multiple of 8 but not of 256; the
+// last tile row / column loads clamped operand rows and stores what exists.
+template <bool AK, bool BKM, typename TC, int EPI, int HLD = 0, bool EDGE = false>
 __global__ __launch_bounds__(kPkThreads) void gemm_pk(TC* C, const bf16* A, const bf16* B, int64_t M, int64_t N,
                                                      int64_t lda, int64_t ldb, int64_t ldc, int64_t kps,
                                                      int64_t splits, float* partial, const void* aux, void* aux_out,
@@ -554,7 +558,8 @@ __global__ __launch_bounds__(kPkThreads) void gemm_pk(TC* C, const bf16* A, cons
     // four values), and the epilogue stages bf16 instead of fp32 (see below)
     constexpr bool SW = std::is_same<TC, bf16>::value && (EPI == EPI_STORE || EPI == EPI_RELU2 || EPI == EPI_SOFTCAP ||
                                                           EPI == EPI_QKV || EPI == EPI_DOUT_D);
-    const int tiles_n = (int)(N / 256), tiles_mn = (int)(M / 256) * tiles_n, items = tiles_mn * (int)splits;
+    static_assert(!EDGE || !HL, "head epilogues take whole tiles");
+    const int tiles_n = (int)((N + 255) / 256), tiles_mn = (int)((M + 255) / 256) * tiles_n, items = tiles_mn * (int)splits;
     const int grid = (int)gridDim.x, b = (int)blockIdx.x;
     const int nk = (int)(kps / kPkBK);
     const int nmine = (items - b + grid - 1) / grid;
@@ -577,6 +582,11 @@ __global__ __launch_bounds__(kPkThreads) void gemm_pk(TC* C, const bf16* A, cons
             const int64_t k0 = (int64_t)z * kps;
             pa = reinterpret_cast<const char*>(A) + 2 * (AK ? (int64_t)tm * 256 * lda + k0 : k0 * lda + tm * 256);
             pb = reinterpret_cast<const char*>(B) + 2 * (BKM ? (int64_t)tn * 256 * ldb + k0 : k0 * ldb + tn * 256);
+            if constexpr (EDGE) {
+                const int ml = (int)M - tm * 256, nl = (int)N - tn * 256;
+                pk_offsets<AK>(aoffs, (int)lda, wave, lane, ml < 256 ? ml : 256);
+                pk_offsets<BKM>(boffs, (int)ldb, wave, lane, nl < 256 ? nl : 256);
+            }
         }
         const unsigned st = lds0 + (g & 1) * kPkStage;
 #pragma unroll
@@ -666,6 +676,7 @@ __global__ __launch_bounds__(kPkThreads) void gemm_pk(TC* C, const bf16* A, cons
         // this wave's block: element (r, c) at base + r * ld + c
         const int64_t cbase = row0 * ldc + col0;
         const int clo = lrow * (int)ldc + lcol;
+        const int mleft = EDGE ? (int)(M - row0) : 0, nleft = EDGE ? (int)(N - col0) : 0;  // rows, columns that exist
         if constexpr (SW) {
             // Per 32-row block i: the lane's 32 values (row m = lane % 32,
             // columns j * 32 + 8 g + 4 (lane / 32) + 0..3) go through the
@@ -815,7 +826,7 @@ __global__ __launch_bounds__(kPkThreads) void gemm_pk(TC* C, const bf16* A, cons
                         // row many times, so keeping them in the caches pays; other
                         // outputs stream past L2 (nontemporal)
                         if constexpr (EPI == EPI_QKV) *qd = q;
-                        else __builtin_nontemporal_store(q, qd);
+                        else if (!EDGE || (rr < mleft - i * 32 - p * 8 && c16 * 8 < nleft - jp * 64)) __builtin_nontemporal_store(q, qd);
                     }
                     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
                     __builtin_amdgcn_wave_barrier();
@@ -834,12 +845,19 @@ __global__ __launch_bounds__(kPkThreads) void gemm_pk(TC* C, const bf16* A, cons
         // pre-activation) is loaded one half strip ahead, into a two-slot
         // register ring, so its latency hides behind the previous strip.
         float4 pre[2][PRE ? 4 : 1];
+        // lanes past the last column count as past the last row
+        const int elrow = EDGE && lcol >= nleft ? 1 << 30 : lrow;
+        auto exists = [&](int s, int t) { return !EDGE || elrow < mleft - s * 16 - t * 4; };
+        // partial sums: this wave's block of split z, and the lane's offset in it
+        float* const pbase = EPI == EPI_PARTIAL ? partial + ((int64_t)z * M + row0) * N + col0 : nullptr;
+        const int plo = lrow * (int)N + lcol;
         auto load_pre = [&](int s, float4 (&dst)[PRE ? 4 : 1]) {
             if constexpr (PRE) {
                 const int64_t rb = cbase + (int64_t)(s * 16) * ldc;
 #pragma unroll
                 for (int t = 0; t < 4; ++t) {
                     const int64_t o = rb + (int64_t)(t * 4) * ldc + clo;
+                    if (!exists(s, t)) continue;
                     if constexpr (EPI == EPI_ACCUM) dst[t] = ld4(C + o);
                     else if constexpr (EPI == EPI_ADD) dst[t] = ld4(static_cast<const float*>(aux) + o);
                     else dst[t] = ld4(static_cast<const TC*>(aux) + o);
@@ -870,9 +888,9 @@ __global__ __launch_bounds__(kPkThreads) void gemm_pk(TC* C, const bf16* A, cons
                     const int r = t * 4 + lrow;
                     const float4 x = *reinterpret_cast<const float4*>(strip + r * 64 + (lcol ^ (((r >> 2) & 1) << 5)));
                     const int64_t o = rb + (int64_t)(t * 4) * ldc + clo;
+                    if (!exists(s, t)) continue;
                     if constexpr (EPI == EPI_PARTIAL) {
-                        const int64_t row = row0 + i * 32 + h * 16 + r;
-                        st4nt(partial + ((int64_t)z * M + row) * N + col0 + lcol, x);
+                        st4nt(pbase + (int64_t)(s * 16 + t * 4) * N + plo, x);
                     } else if constexpr (EPI == EPI_STORE) {
                         st4nt(C + o, x);
                     } else if constexpr (EPI == EPI_ACCUM || EPI == EPI_ADD) {
@@ -1247,16 +1265,19 @@ static int32_t gemm_launch_t(hipStream_t st, TC* C, const TA* A, const TB* B, in
 }
 
 // ---- persistent bf16-operand GEMM (gemm_pk) ----
-// GEMM-space shapes it takes: whole 256 x 256 tiles, 64-deep k-tiles, 16-byte
-// aligned operands whose rows start on 16-byte boundaries.
+// GEMM-space shapes it takes: 256 x 256 tiles (pk_shape: whole ones; pk_pays:
+// with edge tiles), 64-deep k-tiles, 16-byte aligned operands whose rows start
+// on 16-byte boundaries.
 static bool pk_shape(int64_t gm, int64_t gn, int64_t gk) {
     return gm > 0 && gn > 0 && gk > 0 && gm % 256 == 0 && gn % 256 == 0 && gk % kPkBK == 0;
 }
+static int64_t pk_tiles(int64_t gm, int64_t gn) { return ((gm + 255) / 256) * ((gn + 255) / 256); }
+static bool pk_pays(int64_t gm, int64_t gn, int64_t gk, int64_t splits);
 static bool pk_ok(int64_t gm, int64_t gn, int64_t gk, int64_t lda, int64_t ldb, int64_t ldc, const void* A,
-                  const void* B, const void* C) {
+                  const void* B, const void* C, bool edge = true, int64_t splits = 1) {
     // per-lane DMA / epilogue offsets and item indices are 32-bit
-    const bool fits = lda < (1 << 22) && ldb < (1 << 22) && ldc < (1 << 22) && (gm / 256) * (gn / 256) * gk / kPkBK < (1ll << 30);
-    return fits && pk_shape(gm, gn, gk) && lda % 8 == 0 && ldb % 8 == 0 && ldc % 4 == 0 &&
+    const bool fits = lda < (1 << 22) && ldb < (1 << 22) && ldc < (1 << 22) && pk_tiles(gm, gn) * gk / kPkBK < (1ll << 30);
+    return fits && (pk_shape(gm, gn, gk) || (edge && pk_pays(gm, gn, gk, splits))) && lda % 8 == 0 && ldb % 8 == 0 && ldc % 4 == 0 &&
            ((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(B) | reinterpret_cast<uintptr_t>(C)) & 15) == 0;
 }
 static int pk_cus() {
@@ -1282,6 +1303,25 @@ static int64_t pk_splits(int64_t tiles, int64_t gk) {
     return s;
 }
 
+// Whether edge tiles pay: at least half of the persistent grid's rounds must
+// go to elements that exist (the rest is clamped rows, or no item).  Against
+// gemm_k (us, bf16 storage): NT 8192 x 1152 x 384 (0.56 of the rounds) 21.7 ->
+// 13.6, NN 16384 x 640 x 2560 (0.62) 96 -> 73, TN 2560 x 640 x 16384 (0.78)
+// 111 -> 77, 1536 x 384 x 32768 (0.56) 94 -> 68; where 0.30 of the rounds
+// would be useful (NT 5000 x 1000 x 1024) gemm_k's 23.4 beat 24.8.
+static bool pk_pays(int64_t gm, int64_t gn, int64_t gk, int64_t splits) {
+    if (gm < 8 || gn < 8 || gk < kPkBK || gm >= (1 << 30) || gn >= (1 << 30) || gm % 8 != 0 || gn % 8 != 0 || gk % kPkBK != 0) return false;
+    const int64_t cus = pk_cus(), rounds = cdiv(pk_tiles(gm, gn) * splits, cus);
+    return 2 * gm * gn * splits >= rounds * cus * 256 * 256;
+}
+// Splits of a TN product with edge tiles: pk_splits', within the caller's
+// (whose count, gemm_k's, sized the scratch).
+static int64_t pk_edge_splits(int64_t gm, int64_t gn, int64_t gk, int64_t splits) {
+    int64_t s = pk_splits(pk_tiles(gm, gn), gk);
+    while (s > splits) s /= 2;
+    return s;
+}
+
 // C (+)= A . B^T in GEMM space with gemm_pk (operands checked by pk_ok).
 // epi < 0: STORE / ACCUM by `accumulate`, split over the reduction when
 // splits > 1 (fp32 partials in `partial`, then an in-order reduce).
@@ -1291,10 +1331,28 @@ static int32_t pk_launch(hipStream_t st, TC* C, const bf16* A, const bf16* B, in
                          int epi, const void* aux, void* aux_out, float cap, const char* nm) {
     if (splits < 1) splits = 1;
     if (gk % (splits * kPkBK) != 0) return set_error(AR_EINVAL, "%s: split %lld does not divide K", nm, (long long)splits);
-    const int64_t kps = gk / splits, items = (gm / 256) * (gn / 256) * splits;
+    const int64_t kps = gk / splits, items = pk_tiles(gm, gn) * splits;
+    const bool edge = !pk_shape(gm, gn, gk);
     const int cus = pk_cus();
     const unsigned grid = (unsigned)(items < cus ? items : cus);
-#define AR_PK(E)                                                                                                      do {                                                                                                                  static bool attr_set = false;                                                                                     if (!attr_set) {                                                                                                      if (hipFuncSetAttribute((const void*)gemm_pk<AK, BKM, TC, E>,                                                                              hipFuncAttributeMaxDynamicSharedMemorySize, kPkLds) != hipSuccess)                            return set_error(AR_EHIP, "%s: cannot set the LDS size", nm);                                                 attr_set = true;                                                                                              }                                                                                                                 gemm_pk<AK, BKM, TC, E><<<grid, kPkThreads, kPkLds, st>>>(C, A, B, gm, gn, lda, ldb, ldc, kps, splits,                                                                       partial, aux, aux_out, cap, PkHead{});                         } while (0)
+#define AR_PK1(E, ED)                                                                                            \
+    do {                                                                                                         \
+        static bool attr_set = false;                                                                            \
+        if (!attr_set) {                                                                                         \
+            if (hipFuncSetAttribute((const void*)gemm_pk<AK, BKM, TC, E, 0, ED>,                                 \
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, kPkLds) != hipSuccess)           \
+                return set_error(AR_EHIP, "%s: cannot set the LDS size", nm);                                    \
+            attr_set = true;                                                                                     \
+        }                                                                                                        \
+        gemm_pk<AK, BKM, TC, E, 0, ED><<<grid, kPkThreads, kPkLds, st>>>(C, A, B, gm, gn, lda, ldb, ldc, kps,    \
+                                                                         splits, partial, aux, aux_out, cap,     \
+                                                                         PkHead{});                              \
+    } while (0)
+#define AR_PK(E)                                                                                                 \
+    do {                                                                                                         \
+        if (edge) AR_PK1(E, true);                                                                               \
+        else AR_PK1(E, false);                                                                                   \
+    } while (0)
     if (epi >= 0) {
         if (splits != 1) return set_error(AR_EINVAL, "%s: fused epilogues take no reduction split", nm);
         if constexpr (AK) {  // fused epilogues exist for the NT and NN layouts only
@@ -1318,6 +1376,7 @@ static int32_t pk_launch(hipStream_t st, TC* C, const bf16* A, const bf16* B, in
     if (!partial) return set_error(AR_EINVAL, "%s: split-K scratch missing", nm);
     AR_PK(EPI_PARTIAL);
 #undef AR_PK
+#undef AR_PK1
     splitk_reduce<TC>(st, C, partial, gm, gn, ldc, splits, accumulate, 1, 0);
     return check_launch(nm);
 }
@@ -1391,7 +1450,7 @@ bool gemm_head_fusable(int64_t M, int64_t C, int64_t hd) {
 int32_t gemm_qkv_fused(hipStream_t st, bf16* q, bf16* k, bf16* v, const bf16* xn, const bf16* w, int64_t M, int64_t C,
                        int64_t hd, const float* cos_t, const float* sin_t, int64_t period, const float* gate,
                        const float* table, const int64_t* idx) {
-    if (!((hd == 64 || hd == 128) && C % 256 == 0 && period > 0 && pk_ok(M, 3 * C, C, C, C, C, xn, w, q) &&
+    if (!((hd == 64 || hd == 128) && C % 256 == 0 && period > 0 && pk_ok(M, 3 * C, C, C, C, C, xn, w, q, false) &&
           ((reinterpret_cast<uintptr_t>(k) | reinterpret_cast<uintptr_t>(v)) & 15) == 0))
         return AR_EUNSUPPORTED;
     PkHead hx{};
@@ -1410,7 +1469,7 @@ int32_t gemm_qkv_fused(hipStream_t st, bf16* q, bf16* k, bf16* v, const bf16* xn
 
 int32_t gemm_dout_d_fused(hipStream_t st, bf16* dout, float* d, const bf16* gy, const bf16* wt, const float* o,
                           int64_t M, int64_t C, int64_t hd) {
-    if (!((hd == 64 || hd == 128) && pk_ok(M, C, C, C, C, C, gy, wt, dout) &&
+    if (!((hd == 64 || hd == 128) && pk_ok(M, C, C, C, C, C, gy, wt, dout, false) &&
           (reinterpret_cast<uintptr_t>(o) & 15) == 0))
         return AR_EUNSUPPORTED;
     PkHead hx{};
@@ -1526,9 +1585,10 @@ static int32_t gemm_typed(hipStream_t st, int layout, TC* C, const TX* X, const 
         if (layout == 1 && pk_ok(M, K, N, N, K, K, X, W, C))
             return pk_launch<true, false, TC>(st, C, X, W, M, K, N, N, K, K, accumulate, 1, nullptr, -1, nullptr,
                                               nullptr, 0.f, "linear_bwd_dx");
-        if (layout == 2 && pk_ok(N, K, M, N, K, K, X, W, C)) {
-            const int64_t s = splits >= 1 ? splits : pk_splits((N / 256) * (K / 256), M);
-            if (M % (s * kPkBK) == 0)
+        if (layout == 2) {
+            int64_t s = splits >= 1 ? splits : gemm_auto_splits(2, true, true, M, N, K);
+            if (!pk_shape(N, K, M)) s = pk_edge_splits(N, K, M, s);
+            if (M % (s * kPkBK) == 0 && pk_ok(N, K, M, N, K, K, X, W, C, true, s))
                 return pk_launch<false, false, TC>(st, C, X, W, N, K, M, N, K, K, accumulate, s, partial, -1, nullptr,
                                                    nullptr, 0.f, "linear_bwd_dw");
         }
