@@ -88,3 +88,24 @@ def test_softcap_limits(env):
     got = y.tolist()
     assert got[:4] == [0.0, 0.0, 15.0, -15.0] and math.copysign(1, got[1]) == -1
     assert math.isnan(got[4]) and got[5:7] == [15.0, -15.0] and abs(got[7] - 3e-39) < 1e-43
+
+
+# vectors of 4 in batches of 4 per thread of a 512 x 256 grid: one value, a
+# remainder alone, both sides of a whole round of the grid, an odd batch count
+@pytest.mark.parametrize("n", [1, 3, 4, 7, 1025, 524288, 2097151, 2097152, 2097157, 6815749])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_fixed_sums_vs_fp64(env, n, shift):
+    torch, ops = env
+    g = torch.Generator(device="cuda")
+    g.manual_seed(n)
+    a, b = (torch.randn(n + 1, generator=g, device="cuda")[shift:shift + n] for _ in range(2))
+    dot, mean = torch.full((3,), 2.0, device="cuda"), torch.zeros(1, device="cuda")
+    ops.scalar_grad_reduce(dot, a, b, 1, n)
+    ops.mean_reduce(mean, a, n)
+    a64, b64 = a.double(), b.double()
+    # a value passes fewer than 64 roundings: its thread's sum, then the
+    # trees of a block and of the blocks
+    eps = 64 * 2.0 ** -24
+    assert abs(dot[1].item() - 2.0 - (a64 * b64).sum().item()) <= eps * ((a64 * b64).abs().sum().item() + 2.0)
+    assert abs(mean.item() - a64.mean().item()) <= eps * a64.abs().mean().item()
+    assert dot[0].item() == 2.0 and dot[2].item() == 2.0
