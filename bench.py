@@ -39,7 +39,7 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 PEAK_BF16_TFLOPS = 2516.6   # dense bf16 MFMA, MI355X
-PEAK_FP32_TFLOPS = 157.3    # fp32 matrix, MI355X
+PEAK_FP32_TFLOPS = 419.4    # six bf16 products for each fp32 one (three-term splits)
 METRIC = "training tokens/sec @ depth8 d512 T2048 (1 GPU) + MFMA util %"
 CLASS_NAMES = ["linear_fwd", "linear_bwd_dx", "linear_bwd_dw", "flash_attn_fwd", "flash_attn_bwd_dq",
                "flash_attn_bwd_dkv", "muon_polar_express"]
