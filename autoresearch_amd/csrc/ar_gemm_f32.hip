@@ -10,13 +10,21 @@
 // times: norm-wise error against fp64 1.3e-7 at 512^3 (N(0, 1) operands) where
 // the fp32 instruction gave 4.1e-7.
 //
-// Inputs outside that argument are formed on the fp32 matrix cores (redo_fp32,
-// per block), so they give what fp32 products give:
-//   * an infinity or NaN, or a finite value that bf16 rounds to infinity (above
-//     3.39e38), makes every output it touches non-finite, which the block sees;
-//   * a row whose values are all below 2^-110 (7.7e-34) without being zero has
-//     low terms below bf16's least magnitude 2^-133; every thread keeps the
-//     largest magnitude of the row parts it stages.
+// The split is exact for zero and for magnitudes from 2^-110 to 3.39e38; what
+// lies outside is formed on the fp32 matrix cores (fp32_block), per block:
+//   * an infinity or NaN, or a finite value that bf16 rounds to infinity, makes
+//     every output it touches non-finite, which the block sees;
+//   * a value below 2^-110 (7.7e-34) loses up to 2^-134 (half of bf16's least
+//     magnitude), so a sum of R products moves by at most R 2^-134 (max|a| +
+//     max|b|).  With both maxima at 2^24 or less and R at 2^25 or less that is
+//     2^-24 of any output of 2^-60 or more.  A block with a smaller output that
+//     no row of zeros explains, or with a larger operand, looks for such values
+//     and is formed again where it holds one.
+// Muon meets them: the momentum of a row without gradient decays into the
+// subnormals and stays there.  One step of a 2048 x 512 matrix with 2 % of rows
+// at 1e-36 takes 294 us where an ordinary one
+// takes 213 (unstaged scalar loads of the whole block, and no regard to what the
+// outputs are: 484).
 //
 // Layout of a product (GEMM space): C[m, n] (+)= sum_r A(m, r) B(n, r), each
 // operand K-major (r contiguous) or MN-major (m / n contiguous).
@@ -135,13 +143,17 @@ struct X3Load {
             }
         }
     }
-    // A row's values seen here are all below 2^-110 and not all zero: bf16 has
-    // no bits for their low terms (its least magnitude is 2^-133).
-    __device__ __forceinline__ bool tiny() const {
-        bool t = false;
+    __device__ __forceinline__ bool large() const {
+        float m = 0.f;
 #pragma unroll
-        for (const float m : mx) t |= __float_as_uint(m) - 1u < 0x08800000u - 1u;
-        return t;
+        for (const float x : mx) m = fmaxf(m, x);
+        return m > 0x1p24f;
+    }
+    // folds mx into the block's largest magnitude of each row (bit patterns)
+    __device__ __forceinline__ void row_max(unsigned* most) const {
+#pragma unroll
+        for (int i = 0; i < (KMAJ ? NP : 8); ++i)
+            atomicMax(most + (KMAJ ? item(i) / U : (item(0) % C8) * 8 + i), __float_as_uint(mx[i]));
     }
     // the ragged end of the rows lies in this block
     __device__ __forceinline__ bool ragged() const { return !KMAJ && (rows & 7) != 0; }
@@ -239,41 +251,121 @@ __device__ __forceinline__ bf16x8 x3frag(const unsigned char* plane, int r0, int
 
 __device__ __forceinline__ int acc_row(int v, int lane) { return (v >> 2) * 8 + (lane >> 5) * 4 + (v & 3); }
 
-// A wave's block on the fp32 matrix cores, operands straight from memory: only
-// for blocks whose split product came out non-finite.
-template <bool AK, bool BKM, int TM, int TN>
-__device__ __forceinline__ void redo_fp32(f32x16 (&acc)[TM][TN], const float* A, const float* B, int64_t lda,
-                                          int64_t ldb, int64_t M, int64_t N, int64_t row0,
-                                          int64_t col0, int64_t kbeg, int64_t kend) {
-    const int lane = threadIdx.x % kWave;
+constexpr unsigned kTinyBits = 0x08800000u;  // 2^-110
+
+// Whether the block's part of an operand (rows x [kbeg, kend)) holds a value
+// below 2^-110 that is not zero.
+template <bool KMAJ, int ROWS, int THREADS>
+__device__ __forceinline__ bool holds_tiny(const float* g, int64_t ld, int64_t row0, int64_t extent, int64_t kbeg,
+                                           int64_t kend) {
+    constexpr int W = KMAJ || ROWS >= kWave ? kWave : ROWS;  // lanes along what is contiguous
+    const int64_t rows = extent - row0 < ROWS ? extent - row0 : ROWS;
+    const int64_t outer = KMAJ ? rows : kend - kbeg, inner = KMAJ ? kend - kbeg : rows;
+    const float* const s = g + (KMAJ ? row0 * ld + kbeg : kbeg * ld + row0);
+    const int tid = threadIdx.x;
+    unsigned least = ~0u;
+    auto see = [&](float x) __attribute__((always_inline)) {
+        const unsigned u = __float_as_uint(x) * 2u - 1u;  // zero of either sign wraps to the top
+        least = u < least ? u : least;
+    };
+#pragma unroll 4
+    for (int64_t o = tid / W; o < outer; o += THREADS / W) {
+        const float* const q = s + o * ld;
+        if constexpr (KMAJ) {
+#pragma unroll 8
+            for (int64_t i = tid % W; i < inner; i += W) see(q[i]);
+        } else {
+#pragma unroll
+            for (int i = tid % W; i < ROWS; i += W)
+                if (i < inner) see(q[i]);
+        }
+    }
+    return least < kTinyBits * 2u - 1u;
+}
+
+// Eight values of an operand fragment of fp32_block: row r, k-values k .. k + 7
+// (TAIL: those at or past kend are zero).
+template <bool KMAJ, bool TAIL>
+__device__ __forceinline__ void x8(float (&v)[8], const float* g, int64_t ld, int64_t r, int64_t k, int64_t kend) {
+    if constexpr (KMAJ && !TAIL) {
+        const f32x4u a = *reinterpret_cast<const f32x4u*>(g + r * ld + k), b = *reinterpret_cast<const f32x4u*>(g + r * ld + k + 4);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            v[e] = a[e];
+            v[4 + e] = b[e];
+        }
+    } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const int64_t kk = TAIL && k + e >= kend ? kend - 1 : k + e;
+            const float x = KMAJ ? g[r * ld + kk] : g[kk * ld + r];
+            v[e] = TAIL && k + e >= kend ? 0.f : x;
+        }
+    }
+}
+
+// A wave's block on the fp32 matrix cores, straight from memory: every kg-th of
+// KG 16-deep k-steps, each loaded while the one before is multiplied.  Lane half
+// h holds k-values 8 h .. 8 h + 7 of a step; instruction e takes value e of both.
+template <bool AK, bool BKM, int TM, int TN, int KG>
+__device__ __forceinline__ void fp32_block(f32x16 (&acc)[TM][TN], const float* A, const float* B, int64_t lda,
+                                           int64_t ldb, int64_t M, int64_t N, int64_t row0, int64_t col0, int64_t kbeg,
+                                           int64_t kend, int kg) {
+    const int lane = threadIdx.x % kWave, h8 = (lane >> 5) * 8;
+    int64_t ra[TM], rb[TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+        ra[i] = row0 + i * 32 + (lane & 31);
+        ra[i] = ra[i] < M ? ra[i] : M - 1;
+    }
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+        rb[j] = col0 + j * 32 + (lane & 31);
+        rb[j] = rb[j] < N ? rb[j] : N - 1;
+    }
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
         for (int j = 0; j < TN; ++j)
 #pragma unroll
             for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
+    float a[TM][8], b[TN][8];
+    auto load = [&](auto tail_, int64_t k) __attribute__((always_inline)) {
+        constexpr bool TAIL = decltype(tail_)::value;
+#pragma unroll
+        for (int i = 0; i < TM; ++i) x8<AK, TAIL>(a[i], A, lda, ra[i], k + h8, kend);
+#pragma unroll
+        for (int j = 0; j < TN; ++j) x8<BKM, TAIL>(b[j], B, ldb, rb[j], k + h8, kend);
+    };
+    auto mul = [&](const float (&x)[TM][8], const float (&y)[TN][8]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(x[i][e], y[j][e], acc[i][j], 0, 0, 0);
+    };
+    const int64_t whole = (kend - kbeg) / 16, last = kbeg + whole * 16;
+    if (kg < whole) {
+        load(std::false_type{}, kbeg + kg * 16);
 #pragma unroll 1
-    for (int64_t k = kbeg; k < kend; k += 2) {
-        const int64_t kk = k + (lane >> 5), kc = kk < kend ? kk : kend - 1;
-        float a[TM], b[TN];
+        for (int64_t s = kg; s < whole; s += KG) {
+            float x[TM][8], y[TN][8];
 #pragma unroll
-        for (int i = 0; i < TM; ++i) {
-            int64_t r = row0 + i * 32 + (lane & 31);
-            r = r < M ? r : M - 1;
-            const float x = AK ? A[r * lda + kc] : A[kc * lda + r];
-            a[i] = kk < kend ? x : 0.f;
+            for (int e = 0; e < 8; ++e) {
+#pragma unroll
+                for (int i = 0; i < TM; ++i) x[i][e] = a[i][e];
+#pragma unroll
+                for (int j = 0; j < TN; ++j) y[j][e] = b[j][e];
+            }
+            load(std::false_type{}, kbeg + (s + KG < whole ? s + KG : s) * 16);
+            mul(x, y);
         }
-#pragma unroll
-        for (int j = 0; j < TN; ++j) {
-            int64_t c = col0 + j * 32 + (lane & 31);
-            c = c < N ? c : N - 1;
-            const float x = BKM ? B[c * ldb + kc] : B[kc * ldb + c];
-            b[j] = kk < kend ? x : 0.f;
-        }
-#pragma unroll
-        for (int i = 0; i < TM; ++i)
-#pragma unroll
-            for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], b[j], acc[i][j], 0, 0, 0);
+    }
+    if (last < kend && whole % KG == kg) {
+        load(std::true_type{}, last);
+        mul(a, b);
     }
 }
 
@@ -419,8 +511,6 @@ __global__ __launch_bounds__(TL::THREADS, 2) void gemm_x3_k(X3Args p) {
         for (int j = 0; j < TN; ++j)
 #pragma unroll
             for (int v = 0; v < 16; ++v) acc[i][j][v] += low[i][j][v];
-    auto finite = [](float x) { return fabsf(x) <= 3.402823466e38f; };
-    bool bad = la.tiny() || lb.tiny();
     // this wave's block: rows / columns left, and the first element
     const bool part = p.splits > 1;
     const int64_t ldc = part ? p.N : p.ldc;
@@ -433,55 +523,121 @@ __global__ __launch_bounds__(TL::THREADS, 2) void gemm_x3_k(X3Args p) {
         return row < mleft && col < nleft && (!EDGE || (row >= mlow && col >= nlow));
     };
 
-    if constexpr (TL::KG > 1) {
-        // Every group leaves its sums in LDS and then adds, in group order, and
-        // stores 1 / KG of the block: values of 32 x 32 sub-block s / 16, row group s % 16.
-        constexpr int NV = TM * TN * 16, PER = NV / TL::KG;
-        static_assert(NV % TL::KG == 0, "whole values per group");
-        float* const red = reinterpret_cast<float*>(smem_raw) + wq * TL::WM * TL::WN + lane;
+    // Where groups share the reduction, each leaves its sums in LDS and then
+    // adds, in group order, 1 / KG of the block: values of 32 x 32 sub-block
+    // s / 16, row group s % 16.
+    constexpr int NV = TM * TN * 16, PER = NV / TL::KG;
+    static_assert(NV % TL::KG == 0, "whole values per group");
+    float x[TL::KG > 1 ? PER : 1];
+    auto merge = [&]() __attribute__((always_inline)) {
+        if constexpr (TL::KG > 1) {
+            float* const red = reinterpret_cast<float*>(smem_raw) + wq * TL::WM * TL::WN + lane;
 #pragma unroll
-        for (int i = 0; i < TM; ++i)
+            for (int i = 0; i < TM; ++i)
 #pragma unroll
-            for (int j = 0; j < TN; ++j)
+                for (int j = 0; j < TN; ++j)
 #pragma unroll
-                for (int v = 0; v < 16; ++v) red[kg * BM * BN + ((i * TN + j) * 16 + v) * kWave] = acc[i][j][v];
-        __syncthreads();
-        float x[PER];
+                    for (int v = 0; v < 16; ++v) red[kg * BM * BN + ((i * TN + j) * 16 + v) * kWave] = acc[i][j][v];
+            __syncthreads();
 #pragma unroll
-        for (int u = 0; u < PER; ++u) {
-            x[u] = red[(kg * PER + u) * kWave];
+            for (int u = 0; u < PER; ++u) {
+                x[u] = red[(kg * PER + u) * kWave];
 #pragma unroll
-            for (int g = 1; g < TL::KG; ++g) x[u] += red[g * BM * BN + (kg * PER + u) * kWave];
-            bad |= !finite(x[u]);
+                for (int g = 1; g < TL::KG; ++g) x[u] += red[g * BM * BN + (kg * PER + u) * kWave];
+            }
         }
-        if (!__syncthreads_or(bad)) {
+    };
+    // f(value, row, column within the wave's block) of this thread's outputs
+    auto each = [&](auto f) __attribute__((always_inline)) {
+        if constexpr (TL::KG > 1) {
+#pragma unroll
+            for (int u = 0; u < PER; ++u) {
+                const int s = kg * PER + u, ij = s / 16;
+                f(x[u], (ij / TN) * 32 + acc_row(s % 16, lane), (ij % TN) * 32 + (lane & 31));
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j)
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) f(acc[i][j][v], i * 32 + acc_row(v, lane), j * 32 + (lane & 31));
+        }
+    };
+    [[maybe_unused]] auto store = [&]() __attribute__((always_inline)) {
+        // every epilogue operand is read before the first store (C may be aux)
+        if (aux) {
             float y[PER];
+            int n = 0;
+            each([&](float, int row, int col) __attribute__((always_inline)) {
+                y[n++] = own(row, col) ? aux[row * ldc + col] : 0.f;
+            });
 #pragma unroll
-            for (int u = 0; u < PER; ++u) {
-                const int s = kg * PER + u, ij = s / 16;
-                const int row = (ij / TN) * 32 + acc_row(s % 16, lane), col = (ij % TN) * 32 + (lane & 31);
-                y[u] = aux && own(row, col) ? aux[row * ldc + col] : 0.f;
-            }
-#pragma unroll
-            for (int u = 0; u < PER; ++u) {
-                const int s = kg * PER + u, ij = s / 16;
-                const int row = (ij / TN) * 32 + acc_row(s % 16, lane), col = (ij % TN) * 32 + (lane & 31);
-                if (own(row, col)) C[row * ldc + col] = aux ? p.alpha * x[u] + p.beta * y[u] : x[u];
-            }
+            for (int u = 0; u < PER; ++u) x[u] = p.alpha * x[u] + p.beta * y[u];
+        }
+        each([&](float v, int row, int col) __attribute__((always_inline)) {
+            if (own(row, col)) C[row * ldc + col] = v;
+        });
+    };
+    auto any = [](bool b) __attribute__((always_inline)) { return __builtin_amdgcn_readfirstlane(__syncthreads_or(b)) != 0; };
+
+    // An output that is not finite or small, or a large operand; and whether that
+    // is a value outside the split's range.
+    bool inf = false, odd = false;
+    auto odd_block = [&]() __attribute__((always_inline)) {
+        odd = la.large() || lb.large();
+        each([&](float v, int, int) __attribute__((always_inline)) {
+            inf |= !(fabsf(v) <= 3.402823466e38f);
+            odd |= fabsf(v) < 0x1p-60f;
+        });
+        return any(inf || odd);
+    };
+    auto outside = [&]() __attribute__((always_inline)) {
+        if (any(inf)) return true;
+        unsigned* const most = reinterpret_cast<unsigned*>(smem_raw);  // rows of A, then of B
+        for (int i = threadIdx.x; i < BM + BN; i += TL::THREADS) most[i] = 0;
+        __syncthreads();
+        la.row_max(most);
+        lb.row_max(most + BM);
+        __syncthreads();
+        odd = la.large() || lb.large();
+        bool tiny = false;
+        each([&](float v, int row, int col) __attribute__((always_inline)) {
+            const unsigned a = most[wrow + row], b = most[BM + wcol + col];
+            odd |= fabsf(v) < 0x1p-60f && a != 0 && b != 0;
+            tiny |= a - 1u < kTinyBits - 1u || b - 1u < kTinyBits - 1u;
+        });
+        if (!any(odd)) return false;
+        if (any(tiny)) return true;
+        return any(holds_tiny<AK, BM, TL::THREADS>(A, p.lda, m0, p.M, kbeg, kend) ||
+                   holds_tiny<BKM, BN, TL::THREADS>(B, p.ldb, n0, p.N, kbeg, kend));
+    };
+    auto redo = [&]() __attribute__((always_inline)) {
+        fp32_block<AK, BKM, TM, TN, TL::KG>(acc, A, B, p.lda, p.ldb, p.M, p.N, m0 + wrow, n0 + wcol, kbeg, kend, kg);
+    };
+
+    if constexpr (TL::KG > 1) {
+        // Small products: the code they seldom run stays behind their end (in front
+        // of the stores it took a 2048 x 512 x 512 product from 11.4 to 12.5 us).
+        merge();
+        if (!odd_block()) {
+            store();
             return;
         }
-        if (kg > 0) return;  // group 0 forms the whole block again
-    } else {
-#pragma unroll
-        for (int i = 0; i < TM; ++i)
-#pragma unroll
-            for (int j = 0; j < TN; ++j)
-#pragma unroll
-                for (int v = 0; v < 16; ++v) bad |= !finite(acc[i][j][v]);
+        if (outside()) {
+            redo();
+            merge();
+        }
+        store();
+        return;
     }
-    if (TL::KG > 1 || __syncthreads_or(bad))
-        redo_fp32<AK, BKM, TM, TN>(acc, A, B, p.lda, p.ldb, p.M, p.N, m0 + wrow, n0 + wcol, kbeg, kend);
-    // every epilogue operand is read before the first store (C may be aux)
+#pragma unroll 1
+    for (int pass = 0;; ++pass) {
+        if (pass == 1) redo();
+        if (pass == 1 || !odd_block() || !outside()) break;
+    }
+    // as store() does it, written out: through the lambda the 256 x 128 tile
+    // spills 8 to 21 registers (8192 x 2048 x 512 NT 95 -> 100 us)
     if (aux) {
 #pragma unroll
         for (int i = 0; i < TM; ++i)
@@ -587,17 +743,14 @@ int32_t x3_launch(hipStream_t st, const X3Args& p, const char* nm) {
 
 }  // namespace
 
-// Extents the kernel takes: its 8-value loads need 8 values of every stored
-// row (and of the reduction, where an operand is K-major).
-bool gemm_x3_ok(bool ak, bool bk, int64_t M, int64_t N, int64_t K) {
-    return M > 0 && N > 0 && K > 0 && (ak || M >= 8) && (bk || N >= 8) && (!(ak || bk) || K >= 8);
-}
-
 int32_t gemm_x3(hipStream_t st, bool ak, bool bk, float* C, const float* A, const float* B, int64_t M, int64_t N,
                 int64_t K, int64_t lda, int64_t ldb, int64_t ldc, int64_t max_splits, float* partial,
                 const float* aux, float alpha, float beta, int64_t batch, int64_t sA, int64_t sB, int64_t sC,
                 int64_t* splits, const char* nm) {
-    if (!gemm_x3_ok(ak, bk, M, N, K)) return set_error(AR_EINVAL, "%s: extent below 8", nm);
+    // the 8-value loads need 8 values of every stored row (and of the reduction,
+    // where an operand is K-major)
+    if (!(M > 0 && N > 0 && K > 0 && (ak || M >= 8) && (bk || N >= 8) && (!(ak || bk) || K >= 8)))
+        return set_error(AR_EINVAL, "%s: extent below 8", nm);
     const X3Plan plan = x3_plan(M, N, K, batch, partial ? max_splits : 1);
     X3Args p{C, A, B, M, N, K, lda, ldb, ldc, 0, 1, partial, aux, alpha, beta, sA, sB, sC, (int)batch};
     const int64_t bkk = kX3Cost[plan.tile].bk;

@@ -30,7 +30,6 @@ int32_t gemm_f32_add(hipStream_t st, bool bf16, float* C, const float* X, const 
 // alpha times that + beta aux_b (aux laid out as C; may be C).  With partial
 // set the reduction may be split up to max_splits ways: then *splits > 1 and
 // partial holds [batch][splits][M][N] for the caller to add (aux not applied).
-bool gemm_x3_ok(bool ak, bool bk, int64_t M, int64_t N, int64_t K);
 int32_t gemm_x3(hipStream_t st, bool ak, bool bk, float* C, const float* A, const float* B, int64_t M, int64_t N,
                 int64_t K, int64_t lda, int64_t ldb, int64_t ldc, int64_t max_splits, float* partial,
                 const float* aux, float alpha, float beta, int64_t batch, int64_t sA, int64_t sB, int64_t sC,

@@ -86,3 +86,43 @@ def test_fp32_products_non_finite_and_extreme(env, M, N, K):
             inf = np.isinf(ref32) & ~big
             assert np.array_equal(g[inf], ref32[inf])
     assert float(y[9, 2]) == np.float32(3.3999e38)
+
+
+# GEMM-space sizes that choose each block tile, ragged ones, and a split reduction
+@pytest.mark.parametrize("m,n,r", [(40, 48, 72), (33, 57, 131), (1024, 1000, 64), (2050, 1999, 40), (8192, 2048, 64),
+                                   (64, 72, 20000)])
+@pytest.mark.parametrize("exp,up", [(-109, 100), (-111, 100), (-111, 20), (-118, 20), (-125, 100), (-140, 20), (-140, 100)])
+@pytest.mark.parametrize("mixed", [False, True])
+def test_fp32_products_of_small_values(env, m, n, r, exp, up, mixed):
+    """Operands near 2^exp (below 2^-110 bf16 has no bits for their low terms):
+    as whole rows of one operand, or beside larger values of the same row that
+    meet zeros.  The other operand is scaled by 2^up, to ordinary and to small
+    outputs, and has a row of zeros.  Products and sums are of the same kind as
+    in test_fp32_products_vs_fp64, and so is the bound (the least output, 2^-120,
+    still has all its bits).  Either operand is the small one, in all three layouts."""
+    torch, ops, gu = env
+    g = torch.Generator(device="cuda")
+    g.manual_seed(m + n + r + up - exp)
+    small = torch.randn(m if m < n else n, r, generator=g, device="cuda")
+    other = torch.randn(max(m, n), r, generator=g, device="cuda") * 2.0 ** up
+    other[5] = 0.0
+    if mixed:
+        small[:, 1::2] *= 2.0 ** exp
+        other[:, 0::2] = 0.0
+    else:
+        small[::3] *= 2.0 ** exp
+    for first in (False, True):
+        A, B = (small, other) if first else (other, small)
+        M, N = A.shape[0], B.shape[0]
+        At, Bt = A.T.contiguous(), B.T.contiguous()
+        y, dx, dw = gu.empty(M, N), gu.empty(M, N), torch.zeros(M, N, device="cuda")
+        ops.linear_fwd(y, A, B, M, N, r)
+        ops.linear_bwd_dx(dx, A, Bt, M, r, N)
+        ops.linear_bwd_dw(dw, At, Bt, r, M, N)
+        ref, mass = A.double() @ Bt.double(), A.double().abs() @ Bt.double().abs()
+        for got in (y, dx, dw):
+            assert bool(((got.double() - ref).abs() <= 2.0 ** -24 * (6 * r / 16 + 8) * mass).all())
+            # one random rounding per term: row by row, whatever the rows' magnitudes
+            rows = 1 if first else 0
+            err = (got.double() - ref).norm(dim=rows) / ref.norm(dim=rows).clamp_min(1e-300)
+            assert float(err.max()) <= 2.0 ** -24 * 2 * np.sqrt(r + 8)
