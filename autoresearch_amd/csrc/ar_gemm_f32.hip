@@ -451,6 +451,41 @@ __global__ __launch_bounds__(TL::THREADS, 2) void gemm_x3_k(X3Args p) {
         }
     };
 
+    // this wave's block: rows / columns left, and the first element
+    struct Block {
+        int64_t ldc, mleft, nleft;
+        int mlow, nlow;  // first own row / column
+        float* C;
+        const float* aux;
+        __device__ __forceinline__ bool own(int row, int col) const {
+            return row < mleft && col < nleft && (!EDGE || (row >= mlow && col >= nlow));
+        }
+        __device__ __forceinline__ bool whole() const {
+            return mleft >= TL::WM && nleft >= TL::WN && (!EDGE || (mlow <= 0 && nlow <= 0));
+        }
+    };
+    auto block = [&]() __attribute__((always_inline)) {
+        const bool part = p.splits > 1;
+        const int64_t ldc = part ? p.N : p.ldc, c0 = (m0 + wrow) * ldc + n0 + wcol;
+        return Block{ldc, p.M - m0 - wrow, p.N - n0 - wcol, mskip - wrow, nskip - wcol,
+                     (part ? p.partial + ((int64_t)bt * p.splits + z) * p.M * p.N : p.C + bt * p.sC) + c0,
+                     part || !p.aux ? nullptr : p.aux + bt * p.sC + c0};
+    };
+    // D: the epilogue operand is on its way while the product forms
+    constexpr bool EARLY = TL::KG == 1 && TM * TN == 1;
+    f32x16 old;
+    if constexpr (EARLY) {
+        const Block b = block();
+        if (b.aux && b.whole()) {
+#pragma unroll
+            for (int v = 0; v < 16; ++v) old[v] = b.aux[acc_row(v, lane) * b.ldc + (lane & 31)];
+        } else if (b.aux) {
+#pragma unroll
+            for (int v = 0; v < 16; ++v)
+                old[v] = b.own(acc_row(v, lane), lane & 31) ? b.aux[acc_row(v, lane) * b.ldc + (lane & 31)] : 0.f;
+        }
+    }
+
     la.init(A, p.lda, m0, p.M, kbeg);
     lb.init(B, p.ldb, n0, p.N, kbeg);
     const int64_t klen = kend - kbeg;
@@ -511,17 +546,11 @@ __global__ __launch_bounds__(TL::THREADS, 2) void gemm_x3_k(X3Args p) {
         for (int j = 0; j < TN; ++j)
 #pragma unroll
             for (int v = 0; v < 16; ++v) acc[i][j][v] += low[i][j][v];
-    // this wave's block: rows / columns left, and the first element
-    const bool part = p.splits > 1;
-    const int64_t ldc = part ? p.N : p.ldc;
-    const int64_t c0 = (m0 + wrow) * ldc + n0 + wcol;
-    float* const C = (part ? p.partial + ((int64_t)bt * p.splits + z) * p.M * p.N : p.C + bt * p.sC) + c0;
-    const float* const aux = part || !p.aux ? nullptr : p.aux + bt * p.sC + c0;
-    const int64_t mleft = p.M - m0 - wrow, nleft = p.N - n0 - wcol;
-    const int mlow = mskip - wrow, nlow = nskip - wcol;  // first own row / column
-    auto own = [&](int row, int col) {
-        return row < mleft && col < nleft && (!EDGE || (row >= mlow && col >= nlow));
-    };
+    const Block blk = block();
+    const int64_t ldc = blk.ldc;
+    float* const C = blk.C;
+    const float* const aux = blk.aux;
+    auto own = [&](int row, int col) __attribute__((always_inline)) { return blk.own(row, col); };
 
     // Where groups share the reduction, each leaves its sums in LDS and then
     // adds, in group order, 1 / KG of the block: values of 32 x 32 sub-block
@@ -639,21 +668,30 @@ __global__ __launch_bounds__(TL::THREADS, 2) void gemm_x3_k(X3Args p) {
     // as store() does it, written out: through the lambda the 256 x 128 tile
     // spills 8 to 21 registers (8192 x 2048 x 512 NT 95 -> 100 us)
     if (aux) {
+        if constexpr (EARLY) {
+            low[0][0] = old;
+        } else {
 #pragma unroll
-        for (int i = 0; i < TM; ++i)
+            for (int i = 0; i < TM; ++i)
 #pragma unroll
-            for (int j = 0; j < TN; ++j)
+                for (int j = 0; j < TN; ++j)
 #pragma unroll
-                for (int v = 0; v < 16; ++v) {
-                    const int row = i * 32 + acc_row(v, lane), col = j * 32 + (lane & 31);
-                    low[i][j][v] = own(row, col) ? aux[row * ldc + col] : 0.f;
-                }
+                    for (int v = 0; v < 16; ++v) {
+                        const int row = i * 32 + acc_row(v, lane), col = j * 32 + (lane & 31);
+                        low[i][j][v] = own(row, col) ? aux[row * ldc + col] : 0.f;
+                    }
+        }
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll
             for (int j = 0; j < TN; ++j)
 #pragma unroll
                 for (int v = 0; v < 16; ++v) acc[i][j][v] = p.alpha * acc[i][j][v] + p.beta * low[i][j][v];
+    }
+    if (EARLY && blk.whole()) {
+#pragma unroll
+        for (int v = 0; v < 16; ++v) C[acc_row(v, lane) * ldc + (lane & 31)] = acc[0][0][v];
+        return;
     }
 #pragma unroll
     for (int i = 0; i < TM; ++i)
@@ -672,6 +710,7 @@ using X3T = X3Tile<32, 32, 1, 1, 8, 1>;     // 8 waves, one 32 x 32 each, every 
 using X3S = X3Tile<64, 64, 2, 2, 2, 2>;     // 2 x 4 waves of 32 x 32
 using X3M = X3Tile<128, 128, 4, 2, 1, 2>;   // 8 waves of 32 x 64
 using X3L = X3Tile<256, 128, 4, 2, 1, 2>;   // 8 waves of 64 x 64
+using X3D = X3Tile<64, 64, 2, 2, 1, 2>;     // 4 waves of 32 x 32: short reductions (x3_plan)
 
 // Time of a launch in us: c0 + rounds (e + c2 k), k = the reduction in whole
 // k-tiles / 512, rounds of 256 blocks (one per CU), fitted to products timed on
@@ -690,7 +729,8 @@ struct X3Cost {
     int bm, bn, bk;
     double c0, e, c2;
 };
-constexpr X3Cost kX3Cost[4] = {{32, 32, 128, 1.6, 2.7, 2.9}, {64, 64, 64, 2.5, 3.3, 7.3},
+constexpr int kX3Tiles = 4, kX3D = 4;
+constexpr X3Cost kX3Cost[kX3Tiles] = {{32, 32, 128, 1.6, 2.7, 2.9}, {64, 64, 64, 2.5, 3.3, 7.3},
                                {128, 128, 32, 2.0, 3.2, 22.9}, {256, 128, 32, 2.0, 6.0, 39.9}};
 
 struct X3Plan {
@@ -701,10 +741,19 @@ struct X3Plan {
 // The cheapest tile and split of the reduction (a power of two, at most
 // max_splits; each split at least two k-tiles).  A split costs its partials'
 // way to memory and back at ~4 TB/s and the launch that adds them.
-X3Plan x3_plan(int64_t M, int64_t N, int64_t K, int64_t batch, int64_t max_splits) {
+//
+// A product of a short reduction that fills the chip is bound by its output's
+// way to memory, and there by how many blocks a CU keeps: D's four (one LDS
+// stage each) against the others' one (us, against L or M where it was chosen):
+//   8192 x 4096, C += :    R 16 86 -> 62   R 32 80 -> 51   R 64 88 -> 67   R 96 97 -> 81
+//   8192 x 4096, NT:       R 16 44 -> 38   R 32 42 -> 37   R 48 54 -> 50   (64: 51 -> 55)
+//   2048 x 1024, C += :    R 32 10 -> 8.4  R 96 13 -> 10   (100 with two stages: no gain)
+// With B MN-major and nothing to add, D and L are even.
+X3Plan x3_plan(bool nt, int64_t M, int64_t N, int64_t K, int64_t batch, int64_t max_splits, bool aux) {
+    if (K <= (aux ? 96 : nt ? 48 : 0) && cdiv(M, X3D::BM) * cdiv(N, X3D::BN) * batch >= 256) return X3Plan{kX3D, 1};
     X3Plan best{0, 1};
     double least = 1e30;
-    for (int t = 0; t < 4; ++t) {
+    for (int t = 0; t < kX3Tiles; ++t) {
         const X3Cost& c = kX3Cost[t];
         const double tiles = (double)cdiv(M, c.bm) * cdiv(N, c.bn) * batch;
         for (int64_t s = 1; s <= max_splits && (s == 1 || K / s >= 2 * c.bk); s *= 2) {
@@ -730,7 +779,9 @@ int32_t x3_launch_e(hipStream_t st, const X3Args& p, const char* nm) {
         attr_set = true;
     }
     const int64_t grid = cdiv(p.M, TL::BM) * cdiv(p.N, TL::BN) * p.splits * p.batch;
-    gemm_x3_k<AK, BKM, TL, EDGE><<<(unsigned)grid, TL::THREADS, TL::LDS, st>>>(p);
+    // a reduction of less than two k-tiles uses one stage only
+    const int lds = p.K >= 2 * TL::BK ? TL::LDS : TL::STAGE > TL::RED ? TL::STAGE : TL::RED;
+    gemm_x3_k<AK, BKM, TL, EDGE><<<(unsigned)grid, TL::THREADS, lds, st>>>(p);
     return check_launch(nm);
 }
 
@@ -751,9 +802,9 @@ int32_t gemm_x3(hipStream_t st, bool ak, bool bk, float* C, const float* A, cons
     // where an operand is K-major)
     if (!(M > 0 && N > 0 && K > 0 && (ak || M >= 8) && (bk || N >= 8) && (!(ak || bk) || K >= 8)))
         return set_error(AR_EINVAL, "%s: extent below 8", nm);
-    const X3Plan plan = x3_plan(M, N, K, batch, partial ? max_splits : 1);
+    const X3Plan plan = x3_plan(ak && bk, M, N, K, batch, partial ? max_splits : 1, aux != nullptr);
     X3Args p{C, A, B, M, N, K, lda, ldb, ldc, 0, 1, partial, aux, alpha, beta, sA, sB, sC, (int)batch};
-    const int64_t bkk = kX3Cost[plan.tile].bk;
+    const int64_t bkk = plan.tile == kX3D ? X3D::BK : kX3Cost[plan.tile].bk;
     p.kps = cdiv(cdiv(K, plan.splits), bkk) * bkk;
     p.splits = (int)cdiv(K, p.kps);
     if (splits) *splits = p.splits;
@@ -762,6 +813,7 @@ int32_t gemm_x3(hipStream_t st, bool ak, bool bk, float* C, const float* A, cons
         case 0: return x3_launch<AKv, BKv, X3T>(st, p, nm);         \
         case 1: return x3_launch<AKv, BKv, X3S>(st, p, nm);         \
         case 2: return x3_launch<AKv, BKv, X3M>(st, p, nm);         \
+        case kX3D: return x3_launch<AKv, BKv, X3D>(st, p, nm);      \
         default: return x3_launch<AKv, BKv, X3L>(st, p, nm);        \
     }
     if (ak && bk) AR_X3(true, true)

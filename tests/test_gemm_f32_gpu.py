@@ -28,7 +28,10 @@ def _products(torch, ops, gu, M, N, K, x, w, dy, dw0):
 # that choose the large tiles and a split reduction
 SHAPES = [(8, 8, 8), (9, 9, 9), (32, 32, 128), (33, 31, 129), (64, 64, 64), (65, 63, 71), (1, 40, 24), (128, 128, 32),
           (129, 257, 33), (515, 130, 1999), (2048, 513, 520), (4100, 1031, 96), (8192, 2048, 64), (30, 77, 5001),
-          (7, 300, 5), (4097, 3, 12)]
+          (7, 300, 5), (4097, 3, 12),
+          # short reductions of large outputs: fwd over K, dW over M, one k-tile, a part of one, three
+          (1024, 1031, 8), (1100, 1024, 48), (1030, 1021, 33), (16, 1024, 1024), (9, 1030, 1027), (33, 2050, 1000),
+          (96, 1999, 1030)]
 
 
 @pytest.mark.parametrize("M,N,K", SHAPES)
@@ -89,7 +92,7 @@ def test_fp32_products_non_finite_and_extreme(env, M, N, K):
 
 
 # GEMM-space sizes that choose each block tile, ragged ones, and a split reduction
-@pytest.mark.parametrize("m,n,r", [(40, 48, 72), (33, 57, 131), (1024, 1000, 64), (2050, 1999, 40), (8192, 2048, 64),
+@pytest.mark.parametrize("m,n,r", [(40, 48, 72), (33, 57, 131), (1024, 1000, 64), (1040, 1030, 33), (2050, 1999, 40), (8192, 2048, 64),
                                    (64, 72, 20000)])
 @pytest.mark.parametrize("exp,up", [(-109, 100), (-111, 100), (-111, 20), (-118, 20), (-125, 100), (-140, 20), (-140, 100)])
 @pytest.mark.parametrize("mixed", [False, True])
