@@ -7,9 +7,9 @@
 // row stride H*hd), LSE and D are [B, T, H].  Key kp is visible from query qp
 // iff kp <= qp and (window <= 0 or kp >= qp - window).
 //
-// Work decomposition: a workgroup owns 32 QW rows of one (b, h) -- queries for
-// fwd / dQ, keys for dK / dV -- and its waves walk the 32-row tiles of the
-// other side, wave kg of KG every KG-th tile; at the end the KG partial results
+// Work decomposition: a workgroup owns 32 rows of one (b, h) -- queries for
+// fwd / dQ, keys for dK / dV -- and its four waves walk the 32-row tiles of the
+// other side, wave kg every fourth tile; at the end the four partial results
 // are merged through LDS (the forward's with their softmax maxima).  Short
 // sequences thus still fill the chip: at B 4, T 512, H 4 there are 256
 // workgroups with two or three tiles per wave, where 128-row workgroups that
@@ -43,6 +43,7 @@ namespace {
 
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLn2 = 0.6931471805599453f;
+constexpr int kRows = 32, kWaves = 4, kThreads = kWaves * kWave;  // own rows and waves of a workgroup
 
 __device__ __forceinline__ int acc_row(int v, int lane) { return (v >> 2) * 8 + (lane >> 5) * 4 + (v & 3); }
 
@@ -140,12 +141,12 @@ __device__ __forceinline__ void acc_vals(float (&x)[8], const f32x16& a, int s) 
     for (int e = 0; e < 8; ++e) x[e] = a[8 * s + e];
 }
 
-// Split planes of R rows [row0, row0 + R) of an operand in LDS (K-major units,
-// kslot order), written by the whole workgroup.
-template <int R, int HD>
+// Split planes of the own rows of an operand in LDS (K-major units, kslot
+// order), written by the whole workgroup.
+template <int HD>
 __device__ __forceinline__ void own_planes(unsigned char* planes, const Src& t, int row0, int T) {
-    constexpr int U = HD / 8, PB = R * HD * 2;
-    for (int it = threadIdx.x; it < R * U; it += 256) {
+    constexpr int U = HD / 8, PB = kRows * HD * 2;
+    for (int it = threadIdx.x; it < kRows * U; it += kThreads) {
         const int r = it / U, c = it % U, row = row0 + r;
         float x[8];
         ld8(x, t.base + (int64_t)(row < T ? row : T - 1) * t.rs + c * 8);
@@ -156,20 +157,19 @@ __device__ __forceinline__ void own_planes(unsigned char* planes, const Src& t, 
     }
 }
 
-// The wave's own rows as MFMA columns: row row0 + lane % 32 of src, or its
-// split planes (rows r0.. of the workgroup's R).
+// The own rows as MFMA columns: row row0 + lane % 32 of src, or its split planes.
 struct Own {
     const unsigned char* planes;
-    int r0, row0;
+    int row0;
 };
-template <bool EX, int R, int HD>
+template <bool EX, int HD>
 __device__ __forceinline__ Frag<EX> own_frag(const Own& w, const Src& t, int T, int ks, int lane) {
     if constexpr (EX) {
         float x[8];
         row_vals<true>(x, t, w.row0, T, ks, lane);
         return Frag<true>(x);
     } else {
-        return Frag<false>(w.planes, R * HD * 2, kslot<HD / 8>(w.r0 + (lane & 31), 2 * ks + (lane >> 5)) * 16);
+        return Frag<false>(w.planes, kRows * HD * 2, kslot<HD / 8>(lane & 31, 2 * ks + (lane >> 5)) * 16);
     }
 }
 
@@ -197,14 +197,14 @@ __device__ __forceinline__ void add_tile(f32x16 (&c)[HD / 32], const Src& t, int
 }
 
 // The 32 x 32 block of (streamed rows at row0) . (own rows)^T.
-template <bool EX, int R, int HD>
+template <bool EX, int HD>
 __device__ __forceinline__ f32x16 row_products(const Src& t, int row0, int T, const Own& w, const Src& own, int lane) {
     f32x16 c = zero16(), low = zero16();
 #pragma unroll
     for (int ks = 0; ks < HD / 16; ++ks) {
         float x[8];
         row_vals<EX>(x, t, row0, T, ks, lane);
-        dot16(c, low, Frag<EX>(x), own_frag<EX, R, HD>(w, own, T, ks, lane));
+        dot16(c, low, Frag<EX>(x), own_frag<EX, HD>(w, own, T, ks, lane));
         // two k-steps' loads in flight: with all HD / 16 hoisted dQ spills at hd
         // 128 and every kernel was slower (B16 T2048: fwd 552 -> 530 us, dQ 896 -> 842)
         if (ks & 1) __builtin_amdgcn_sched_barrier(0);
@@ -246,21 +246,21 @@ __device__ __forceinline__ void put_block(float* reg, const f32x16 (&acc)[HD / 3
                 make_float4(acc[dt][g * 4] * f, acc[dt][g * 4 + 1] * f, acc[dt][g * 4 + 2] * f, acc[dt][g * 4 + 3] * f);
 }
 
-// Sums the KG regions of each row (in order), times scale_row[row]; y holds
+// Sums the waves' regions of each row (in order), times scale_row[row]; y holds
 // this thread's float4s.  Returns whether one of a valid row is not finite or
 // below 2^-100.
-template <int HD, int QW, int KG>
-__device__ __forceinline__ bool sum_blocks(float4 (&y)[QW * 32 * HD / 1024], const float* regs, const float* scale_row,
+template <int HD>
+__device__ __forceinline__ bool sum_blocks(float4 (&y)[HD / 32], const float* regs, const float* scale_row,
                                            int valid) {
-    constexpr int RB = 32 * ld_out<HD>();
+    constexpr int RB = kRows * ld_out<HD>();
     bool bad = false;
 #pragma unroll
-    for (int n = 0; n < QW * 32 * HD / 1024; ++n) {
-        const int i = (n * 256 + (int)threadIdx.x) * 4, r = i / HD, d = i % HD;
-        const float* s = regs + (r / 32) * KG * RB + (r % 32) * ld_out<HD>() + d;
+    for (int n = 0; n < HD / 32; ++n) {
+        const int i = (n * kThreads + (int)threadIdx.x) * 4, r = i / HD, d = i % HD;
+        const float* s = regs + r * ld_out<HD>() + d;
         float4 t = *reinterpret_cast<const float4*>(s);
 #pragma unroll
-        for (int g = 1; g < KG; ++g) {
+        for (int g = 1; g < kWaves; ++g) {
             const float4 u = *reinterpret_cast<const float4*>(s + g * RB);
             t = make_float4(t.x + u.x, t.y + u.y, t.z + u.z, t.w + u.w);
         }
@@ -273,19 +273,21 @@ __device__ __forceinline__ bool sum_blocks(float4 (&y)[QW * 32 * HD / 1024], con
     }
     return bad;
 }
-template <int HD, int QW>
-__device__ __forceinline__ void store_blocks(float* out, int64_t rs, const float4 (&y)[QW * 32 * HD / 1024], int valid) {
+template <int HD>
+__device__ __forceinline__ void store_blocks(float* out, int64_t rs, const float4 (&y)[HD / 32], int valid) {
 #pragma unroll
-    for (int n = 0; n < QW * 32 * HD / 1024; ++n) {
-        const int i = (n * 256 + (int)threadIdx.x) * 4, r = i / HD, d = i % HD;
+    for (int n = 0; n < HD / 32; ++n) {
+        const int i = (n * kThreads + (int)threadIdx.x) * 4, r = i / HD, d = i % HD;
         if (r < valid) *reinterpret_cast<float4*>(out + (int64_t)r * rs + d) = y[n];
     }
 }
 
-template <int HD, int QW, int KG, int NP>
+// The planes of NP operands, or the waves' regions; then m and l of every wave and row, and a row of scales.
+constexpr int kStatLds = (2 * kWaves + 1) * kRows * 4;
+template <int HD, int NP>
 constexpr size_t attn_lds() {
-    const size_t planes = (size_t)NP * 3 * QW * 32 * HD * 2, regs = (size_t)QW * KG * 32 * ld_out<HD>() * 4;
-    return (planes > regs ? planes : regs) + (size_t)(2 * QW * KG + QW) * 32 * 4;
+    const size_t planes = (size_t)NP * 3 * kRows * HD * 2, regs = (size_t)kWaves * kRows * ld_out<HD>() * 4;
+    return (planes > regs ? planes : regs) + kStatLds;
 }
 
 // First row of tile t as it is read: split products take whole tiles, so a
@@ -297,7 +299,7 @@ __device__ __forceinline__ int tile_row(int t, int T) {
 }
 
 // ============================ forward ============================
-template <bool EX, int HD, int KG, int R>
+template <bool EX, int HD>
 __device__ __forceinline__ void fwd_tiles(f32x16 (&o)[HD / 32], float& m, float& l, const Own& w, const Src& q,
                                           const Src& k, const Src& v, int T, int window, float scale_log2, int kg,
                                           int lane) {
@@ -310,9 +312,9 @@ __device__ __forceinline__ void fwd_tiles(f32x16 (&o)[HD / 32], float& m, float&
     const int first = window > 0 && qw > window ? (qw - window) / 32 : 0;
     const int last = (qw + 31 < T ? qw + 31 : T - 1) / 32;
 #pragma unroll 1
-    for (int kt = first + kg; kt <= last; kt += KG) {
+    for (int kt = first + kg; kt <= last; kt += kWaves) {
         const int k0 = tile_row<EX>(kt, T);
-        f32x16 s = row_products<EX, R, HD>(k, k0, T, w, q, lane);
+        f32x16 s = row_products<EX, HD>(k, k0, T, w, q, lane);
         float mt = -INFINITY;
         const bool full = kt * 32 + 31 <= qw && (window <= 0 || kt * 32 >= qw + 31 - window);  // no masked pair
 #pragma unroll
@@ -345,67 +347,65 @@ __device__ __forceinline__ void fwd_tiles(f32x16 (&o)[HD / 32], float& m, float&
     }
 }
 
-template <int HD, int QW, int KG>
-__global__ __launch_bounds__(256, 2) void attn_fwd_k(float* out, float* lse, const float* qp, const float* kp,
+template <int HD>
+__global__ __launch_bounds__(kThreads, 2) void attn_fwd_k(float* out, float* lse, const float* qp, const float* kp,
                                                      const float* vp, int T, int H, int nblk, int heads, int window,
                                                      float scale_log2) {
-    constexpr int R = QW * 32;
     extern __shared__ __align__(16) unsigned char smem[];
-    constexpr size_t kMain = attn_lds<HD, QW, KG, 1>() - (size_t)(2 * QW * KG + QW) * 32 * 4;
+    constexpr size_t kMain = attn_lds<HD, 1>() - kStatLds;
     float* const regs = reinterpret_cast<float*>(smem);
     float* const ml = reinterpret_cast<float*>(smem + kMain);  // m, l per wave and row, then 1 / l per row
-    float* const inv = ml + 2 * QW * KG * 32;
-    const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-    const int kg = wave % KG, wq = wave / KG;
+    float* const inv = ml + 2 * kWaves * kRows;
+    const int lane = threadIdx.x % kWave, kg = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     int bh, blk;
     block_of(nblk, heads, true, bh, blk);
-    const int b = bh / H, h = bh % H, q0 = blk * R;
+    const int b = bh / H, h = bh % H, q0 = blk * kRows;
     const int64_t rs = (int64_t)H * HD, off = (int64_t)b * T * rs + (int64_t)h * HD;
     const Src q(qp + off, rs, lane), k(kp + off, rs, lane), v(vp + off, rs, lane);
-    const Own w{smem, wq * 32, q0 + wq * 32};
-    const int valid = T - q0 < R ? T - q0 : R, my_q = w.row0 + lane;
+    const Own w{smem, q0};
+    const int valid = T - q0 < kRows ? T - q0 : kRows, my_q = w.row0 + lane;
 
-    own_planes<R, HD>(smem, q, q0, T);
+    own_planes<HD>(smem, q, q0, T);
     __syncthreads();
     f32x16 o[HD / 32];
     float m, l;
-    if (T >= 32) fwd_tiles<false, HD, KG, R>(o, m, l, w, q, k, v, T, window, scale_log2, kg, lane);
-    float4 y[QW * 32 * HD / 1024];
+    if (T >= 32) fwd_tiles<false, HD>(o, m, l, w, q, k, v, T, window, scale_log2, kg, lane);
+    float4 y[HD / 32];
     float my_lse = 0.f;
 #pragma unroll 1
     for (int pass = T >= 32 ? 0 : 1;; ++pass) {
-        if (pass == 1) fwd_tiles<true, HD, KG, R>(o, m, l, w, q, k, v, T, window, scale_log2, kg, lane);
+        if (pass == 1) fwd_tiles<true, HD>(o, m, l, w, q, k, v, T, window, scale_log2, kg, lane);
         __syncthreads();  // the planes / the first pass's regions are done with
         if (lane < 32) {
-            ml[(wave * 2) * 32 + lane] = m;
-            ml[(wave * 2 + 1) * 32 + lane] = l;
+            ml[(kg * 2) * 32 + lane] = m;
+            ml[(kg * 2 + 1) * 32 + lane] = l;
         }
         __syncthreads();
         float mt = -INFINITY, lt = 0.f;
 #pragma unroll
-        for (int g = 0; g < KG; ++g) mt = fmaxf(mt, ml[((wq * KG + g) * 2) * 32 + (lane & 31)]);
+        for (int g = 0; g < kWaves; ++g) mt = fmaxf(mt, ml[g * 64 + (lane & 31)]);
         const float m_use = mt == -INFINITY ? 0.f : mt;
 #pragma unroll
-        for (int g = 0; g < KG; ++g) {
-            const int i = ((wq * KG + g) * 2) * 32 + (lane & 31);
+        for (int g = 0; g < kWaves; ++g) {
+            const int i = g * 64 + (lane & 31);
             lt += ml[i + 32] * exp2_hw(ml[i] - m_use);
         }
-        put_block<HD>(regs + wave * 32 * ld_out<HD>(), o, exp2_hw(m - m_use), lane);
+        put_block<HD>(regs + kg * kRows * ld_out<HD>(), o, exp2_hw(m - m_use), lane);
         if (kg == 0 && lane < 32) {
-            inv[wq * 32 + lane] = lt > 0.f ? 1.0f / lt : 0.f;
+            inv[lane] = lt > 0.f ? 1.0f / lt : 0.f;
             my_lse = lt > 0.f ? (mt + log2f(lt)) * kLn2 : -INFINITY;
         }
         __syncthreads();
-        bool bad = sum_blocks<HD, QW, KG>(y, regs, inv, valid);
+        bool bad = sum_blocks<HD>(y, regs, inv, valid);
         bad |= kg == 0 && lane < 32 && my_q < T && !(fabsf(my_lse) <= 3.402823466e38f);
         if (!__syncthreads_or(bad) || pass == 1) break;
     }
-    store_blocks<HD, QW>(out + off + (int64_t)q0 * rs, rs, y, valid);
+    store_blocks<HD>(out + off + (int64_t)q0 * rs, rs, y, valid);
     if (kg == 0 && lane < 32 && my_q < T) lse[((int64_t)b * T + my_q) * H + h] = my_lse;
 }
 
 // ============================ backward: dQ ============================
-template <bool EX, int HD, int KG, int R>
+template <bool EX, int HD>
 __device__ __forceinline__ void dq_tiles(f32x16 (&acc)[HD / 32], const Own& w, const Src& q, const Src& k, const Src& v,
                                          const Src& dout, int T, int window, float scale_log2, float lse2, float dd,
                                          int kg, int lane) {
@@ -413,14 +413,14 @@ __device__ __forceinline__ void dq_tiles(f32x16 (&acc)[HD / 32], const Own& w, c
     for (int dt = 0; dt < HD / 32; ++dt) acc[dt] = zero16();
     const int qw = w.row0, my_q = qw + (lane & 31);
     if (qw >= T) return;
-    const Own wd{w.planes + 3 * R * HD * 2, w.r0, w.row0};  // Q planes, then dO planes
+    const Own wd{w.planes + 3 * kRows * HD * 2, w.row0};  // Q planes, then dO planes
     const int first = window > 0 && qw > window ? (qw - window) / 32 : 0;
     const int last = (qw + 31 < T ? qw + 31 : T - 1) / 32;
 #pragma unroll 1
-    for (int kt = first + kg; kt <= last; kt += KG) {
+    for (int kt = first + kg; kt <= last; kt += kWaves) {
         const int k0 = tile_row<EX>(kt, T);
-        const f32x16 s = row_products<EX, R, HD>(k, k0, T, w, q, lane);
-        f32x16 ds = row_products<EX, R, HD>(v, k0, T, wd, dout, lane);
+        const f32x16 s = row_products<EX, HD>(k, k0, T, w, q, lane);
+        f32x16 ds = row_products<EX, HD>(v, k0, T, wd, dout, lane);
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
             const int key = k0 + acc_row(e, lane);
@@ -432,46 +432,44 @@ __device__ __forceinline__ void dq_tiles(f32x16 (&acc)[HD / 32], const Own& w, c
     }
 }
 
-template <int HD, int QW, int KG>
-__global__ __launch_bounds__(256, 2) void attn_dq_k(float* dq, const float* qp, const float* kp, const float* vp,
+template <int HD>
+__global__ __launch_bounds__(kThreads, 2) void attn_dq_k(float* dq, const float* qp, const float* kp, const float* vp,
                                                     const float* dop, const float* lse, const float* dbuf, int T, int H,
                                                     int nblk, int heads, int window, float scale_log2, float scale) {
-    constexpr int R = QW * 32;
     extern __shared__ __align__(16) unsigned char smem[];
     float* const regs = reinterpret_cast<float*>(smem);
-    const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-    const int kg = wave % KG, wq = wave / KG;
+    const int lane = threadIdx.x % kWave, kg = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     int bh, blk;
     block_of(nblk, heads, true, bh, blk);
-    const int b = bh / H, h = bh % H, q0 = blk * R;
+    const int b = bh / H, h = bh % H, q0 = blk * kRows;
     const int64_t rs = (int64_t)H * HD, off = (int64_t)b * T * rs + (int64_t)h * HD;
     const Src q(qp + off, rs, lane), k(kp + off, rs, lane), v(vp + off, rs, lane), dout(dop + off, rs, lane);
-    const Own w{smem, wq * 32, q0 + wq * 32};
-    const int valid = T - q0 < R ? T - q0 : R, my_q = w.row0 + (lane & 31);
+    const Own w{smem, q0};
+    const int valid = T - q0 < kRows ? T - q0 : kRows, my_q = w.row0 + (lane & 31);
     const int64_t bth = ((int64_t)b * T + (my_q < T ? my_q : 0)) * H + h;
     const float lse2 = lse[bth] * kLog2e, dd = dbuf[bth];
 
-    own_planes<R, HD>(smem, q, q0, T);
-    own_planes<R, HD>(smem + 3 * R * HD * 2, dout, q0, T);
+    own_planes<HD>(smem, q, q0, T);
+    own_planes<HD>(smem + 3 * kRows * HD * 2, dout, q0, T);
     __syncthreads();
     f32x16 acc[HD / 32];
     if (T >= 32)
-        dq_tiles<false, HD, KG, R>(acc, w, q, k, v, dout, T, window, scale_log2, lse2, dd, kg, lane);
-    float4 y[QW * 32 * HD / 1024];
+        dq_tiles<false, HD>(acc, w, q, k, v, dout, T, window, scale_log2, lse2, dd, kg, lane);
+    float4 y[HD / 32];
 #pragma unroll 1
     for (int pass = T >= 32 ? 0 : 1;; ++pass) {
-        if (pass == 1) dq_tiles<true, HD, KG, R>(acc, w, q, k, v, dout, T, window, scale_log2, lse2, dd, kg, lane);
+        if (pass == 1) dq_tiles<true, HD>(acc, w, q, k, v, dout, T, window, scale_log2, lse2, dd, kg, lane);
         __syncthreads();
-        put_block<HD>(regs + wave * 32 * ld_out<HD>(), acc, scale, lane);
+        put_block<HD>(regs + kg * kRows * ld_out<HD>(), acc, scale, lane);
         __syncthreads();
-        const bool bad = sum_blocks<HD, QW, KG>(y, regs, nullptr, valid);
+        const bool bad = sum_blocks<HD>(y, regs, nullptr, valid);
         if (!__syncthreads_or(bad) || pass == 1) break;
     }
-    store_blocks<HD, QW>(dq + off + (int64_t)q0 * rs, rs, y, valid);
+    store_blocks<HD>(dq + off + (int64_t)q0 * rs, rs, y, valid);
 }
 
 // ============================ backward: dK, dV ============================
-template <bool EX, int HD, int KG, int R>
+template <bool EX, int HD>
 __device__ __forceinline__ void dkv_tiles(f32x16 (&dka)[HD / 32], f32x16 (&dva)[HD / 32], const Own& w, const Src& q,
                                           const Src& k, const Src& v, const Src& dout, const float* lse,
                                           const float* dbuf, int H, int T, int window, float scale_log2, int kg,
@@ -480,12 +478,12 @@ __device__ __forceinline__ void dkv_tiles(f32x16 (&dka)[HD / 32], f32x16 (&dva)[
     for (int dt = 0; dt < HD / 32; ++dt) dka[dt] = dva[dt] = zero16();
     const int kw = w.row0, my_k = kw + (lane & 31);
     if (kw >= T) return;
-    const Own wv{w.planes + 3 * R * HD * 2, w.r0, w.row0};  // K planes, then V planes
+    const Own wv{w.planes + 3 * kRows * HD * 2, w.row0};  // K planes, then V planes
     const int qlast = window > 0 && kw + 31 + window < T ? kw + 31 + window : T - 1;
 #pragma unroll 1
-    for (int qt = kw / 32 + kg; qt <= qlast / 32; qt += KG) {
+    for (int qt = kw / 32 + kg; qt <= qlast / 32; qt += kWaves) {
         const int q0 = tile_row<EX>(qt, T);
-        f32x16 p = row_products<EX, R, HD>(q, q0, T, w, k, lane);
+        f32x16 p = row_products<EX, HD>(q, q0, T, w, k, lane);
         float dd[16];
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
@@ -496,7 +494,7 @@ __device__ __forceinline__ void dkv_tiles(f32x16 (&dka)[HD / 32], f32x16 (&dva)[
             p[e] = ok ? exp2_hw(p[e] * scale_log2 - lse[at] * kLog2e) : 0.f;
         }
         add_tile<EX, HD>(dva, dout, q0, T, p, lane);
-        f32x16 ds = row_products<EX, R, HD>(dout, q0, T, wv, v, lane);
+        f32x16 ds = row_products<EX, HD>(dout, q0, T, wv, v, lane);
 #pragma unroll
         for (int e = 0; e < 16; ++e) ds[e] = p[e] * (ds[e] - dd[e]);
         add_tile<EX, HD>(dka, q, q0, T, ds, lane);
@@ -507,48 +505,46 @@ __device__ __forceinline__ void dkv_tiles(f32x16 (&dka)[HD / 32], f32x16 (&dva)[
 // both accumulators, both fragments and their loads in registers) is faster
 // while the grid gives each CU no more than two (B4 T512 H4: 41 against 54 us),
 // two with ~50 spilled registers beyond that (B16 T2048 H4: 1630 against 1900).
-template <int HD, int QW, int KG, int OCC>
-__global__ __launch_bounds__(256, OCC) void attn_dkv_k(float* dk, float* dv, const float* qp, const float* kp,
+template <int HD, int OCC>
+__global__ __launch_bounds__(kThreads, OCC) void attn_dkv_k(float* dk, float* dv, const float* qp, const float* kp,
                                                      const float* vp, const float* dop, const float* lse,
                                                      const float* dbuf, int T, int H, int nblk, int heads, int window,
                                                      float scale_log2, float scale) {
-    constexpr int R = QW * 32;
     extern __shared__ __align__(16) unsigned char smem[];
     float* const regs = reinterpret_cast<float*>(smem);
-    const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-    const int kg = wave % KG, wq = wave / KG;
+    const int lane = threadIdx.x % kWave, kg = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     int bh, blk;
     block_of(nblk, heads, false, bh, blk);
-    const int b = bh / H, h = bh % H, k0 = blk * R;
+    const int b = bh / H, h = bh % H, k0 = blk * kRows;
     const int64_t rs = (int64_t)H * HD, off = (int64_t)b * T * rs + (int64_t)h * HD;
     const Src q(qp + off, rs, lane), k(kp + off, rs, lane), v(vp + off, rs, lane), dout(dop + off, rs, lane);
-    const Own w{smem, wq * 32, k0 + wq * 32};
-    const int valid = T - k0 < R ? T - k0 : R;
+    const Own w{smem, k0};
+    const int valid = T - k0 < kRows ? T - k0 : kRows;
     const float* const lb = lse + (int64_t)b * T * H + h;
     const float* const db = dbuf + (int64_t)b * T * H + h;
 
-    own_planes<R, HD>(smem, k, k0, T);
-    own_planes<R, HD>(smem + 3 * R * HD * 2, v, k0, T);
+    own_planes<HD>(smem, k, k0, T);
+    own_planes<HD>(smem + 3 * kRows * HD * 2, v, k0, T);
     __syncthreads();
     f32x16 dka[HD / 32], dva[HD / 32];
     if (T >= 32)
-        dkv_tiles<false, HD, KG, R>(dka, dva, w, q, k, v, dout, lb, db, H, T, window, scale_log2, kg, lane);
-    float4 yk[QW * 32 * HD / 1024], yv[QW * 32 * HD / 1024];
+        dkv_tiles<false, HD>(dka, dva, w, q, k, v, dout, lb, db, H, T, window, scale_log2, kg, lane);
+    float4 yk[HD / 32], yv[HD / 32];
 #pragma unroll 1
     for (int pass = T >= 32 ? 0 : 1;; ++pass) {
-        if (pass == 1) dkv_tiles<true, HD, KG, R>(dka, dva, w, q, k, v, dout, lb, db, H, T, window, scale_log2, kg, lane);
+        if (pass == 1) dkv_tiles<true, HD>(dka, dva, w, q, k, v, dout, lb, db, H, T, window, scale_log2, kg, lane);
         __syncthreads();
-        put_block<HD>(regs + wave * 32 * ld_out<HD>(), dka, scale, lane);
+        put_block<HD>(regs + kg * kRows * ld_out<HD>(), dka, scale, lane);
         __syncthreads();
-        bool bad = sum_blocks<HD, QW, KG>(yk, regs, nullptr, valid);
+        bool bad = sum_blocks<HD>(yk, regs, nullptr, valid);
         __syncthreads();
-        put_block<HD>(regs + wave * 32 * ld_out<HD>(), dva, 1.0f, lane);
+        put_block<HD>(regs + kg * kRows * ld_out<HD>(), dva, 1.0f, lane);
         __syncthreads();
-        bad |= sum_blocks<HD, QW, KG>(yv, regs, nullptr, valid);
+        bad |= sum_blocks<HD>(yv, regs, nullptr, valid);
         if (!__syncthreads_or(bad) || pass == 1) break;
     }
-    store_blocks<HD, QW>(dk + off + (int64_t)k0 * rs, rs, yk, valid);
-    store_blocks<HD, QW>(dv + off + (int64_t)k0 * rs, rs, yv, valid);
+    store_blocks<HD>(dk + off + (int64_t)k0 * rs, rs, yk, valid);
+    store_blocks<HD>(dv + off + (int64_t)k0 * rs, rs, yv, valid);
 }
 
 template <typename K>
@@ -558,32 +554,32 @@ int32_t attn_attr(K* kern, size_t lds) {
     return AR_OK;
 }
 
-template <int HD, int QW, int KG>
+template <int HD>
 int32_t attn_launch(hipStream_t st, AttnOp op, float* o1, float* o2, const float* q, const float* k, const float* v,
                     const float* dout, const float* lse, const float* dbuf, int B, int T, int H, int window, float sc) {
     const float scale = sc > 0.f ? sc : 1.0f / sqrtf((float)HD), scale_log2 = scale * kLog2e;
-    const int nblk = (int)cdiv(T, QW * 32), heads = B * H;
+    const int nblk = (int)cdiv(T, kRows), heads = B * H;
     const unsigned grid = (unsigned)nblk * (unsigned)heads;
     if (op == AttnOp::FWD) {
-        constexpr size_t lds = attn_lds<HD, QW, KG, 1>();
-        static const int32_t ok = attn_attr(attn_fwd_k<HD, QW, KG>, lds);
+        constexpr size_t lds = attn_lds<HD, 1>();
+        static const int32_t ok = attn_attr(attn_fwd_k<HD>, lds);
         if (ok) return ok;
-        attn_fwd_k<HD, QW, KG><<<grid, 256, lds, st>>>(o1, o2, q, k, v, T, H, nblk, heads, window, scale_log2);
+        attn_fwd_k<HD><<<grid, kThreads, lds, st>>>(o1, o2, q, k, v, T, H, nblk, heads, window, scale_log2);
         return check_launch("flash_attn_fwd");
     }
-    constexpr size_t lds = attn_lds<HD, QW, KG, 2>();
+    constexpr size_t lds = attn_lds<HD, 2>();
     if (op == AttnOp::DQ) {
-        static const int32_t ok = attn_attr(attn_dq_k<HD, QW, KG>, lds);
+        static const int32_t ok = attn_attr(attn_dq_k<HD>, lds);
         if (ok) return ok;
-        attn_dq_k<HD, QW, KG><<<grid, 256, lds, st>>>(o1, q, k, v, dout, lse, dbuf, T, H, nblk, heads, window,
+        attn_dq_k<HD><<<grid, kThreads, lds, st>>>(o1, q, k, v, dout, lse, dbuf, T, H, nblk, heads, window,
                                                       scale_log2, scale);
         return check_launch("flash_attn_bwd_dq");
     }
 #define AR_DKV(OCC)                                                                                                  \
     do {                                                                                                             \
-        static const int32_t ok = attn_attr(attn_dkv_k<HD, QW, KG, OCC>, lds);                                       \
+        static const int32_t ok = attn_attr(attn_dkv_k<HD, OCC>, lds);                                       \
         if (ok) return ok;                                                                                           \
-        attn_dkv_k<HD, QW, KG, OCC><<<grid, 256, lds, st>>>(o1, o2, q, k, v, dout, lse, dbuf, T, H, nblk, heads, window, \
+        attn_dkv_k<HD, OCC><<<grid, kThreads, lds, st>>>(o1, o2, q, k, v, dout, lse, dbuf, T, H, nblk, heads, window, \
                                                             scale_log2, scale);                                      \
     } while (0)
     if constexpr (HD == 128) {
@@ -605,7 +601,7 @@ int32_t attn_f32(hipStream_t st, AttnOp op, float* o1, float* o2, const float* q
     if (B <= 0 || T <= 0 || H <= 0) return B == 0 || T == 0 ? AR_OK : set_error(AR_EINVAL, "flash attention: bad shape");
     if (B * H > 65535 || T > (1 << 30)) return set_error(AR_EINVAL, "flash attention: shape too large");
     const int w = window > T ? (int)T : (int)window;  // a window >= T is full causal
-#define AR_AT(HDv) attn_launch<HDv, 1, 4>(st, op, o1, o2, q, k, v, dout, lse, dbuf, (int)B, (int)T, (int)H, w, scale)
+#define AR_AT(HDv) attn_launch<HDv>(st, op, o1, o2, q, k, v, dout, lse, dbuf, (int)B, (int)T, (int)H, w, scale)
     switch (HD) {
         case 32: return AR_AT(32);
         case 64: return AR_AT(64);
