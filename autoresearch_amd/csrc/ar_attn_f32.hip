@@ -246,12 +246,12 @@ __device__ __forceinline__ void put_block(float* reg, const f32x16 (&acc)[HD / 3
                 make_float4(acc[dt][g * 4] * f, acc[dt][g * 4 + 1] * f, acc[dt][g * 4 + 2] * f, acc[dt][g * 4 + 3] * f);
 }
 
-// Sums the waves' regions of each row (in order), times scale_row[row]; y holds
-// this thread's float4s.  Returns whether one of a valid row is not finite or
+// Sums the regions of each row over the first ng waves (those that had a tile),
+// in order, times scale_row[row]; y holds this thread's float4s.  Returns whether one of a valid row is not finite or
 // below 2^-100.
 template <int HD>
 __device__ __forceinline__ bool sum_blocks(float4 (&y)[HD / 32], const float* regs, const float* scale_row,
-                                           int valid) {
+                                           int valid, int ng) {
     constexpr int RB = kRows * ld_out<HD>();
     bool bad = false;
 #pragma unroll
@@ -261,6 +261,7 @@ __device__ __forceinline__ bool sum_blocks(float4 (&y)[HD / 32], const float* re
         float4 t = *reinterpret_cast<const float4*>(s);
 #pragma unroll
         for (int g = 1; g < kWaves; ++g) {
+            if (g >= ng) break;
             const float4 u = *reinterpret_cast<const float4*>(s + g * RB);
             t = make_float4(t.x + u.x, t.y + u.y, t.z + u.z, t.w + u.w);
         }
@@ -282,7 +283,8 @@ __device__ __forceinline__ void store_blocks(float* out, int64_t rs, const float
     }
 }
 
-// The planes of NP operands, or the waves' regions; then m and l of every wave and row, and a row of scales.
+// The planes of NP operands, or the waves' regions; then two values
+// of every wave and row (m and l; LSE and D), and a row of scales.
 constexpr int kStatLds = (2 * kWaves + 1) * kRows * 4;
 template <int HD, int NP>
 constexpr size_t attn_lds() {
@@ -298,6 +300,18 @@ __device__ __forceinline__ int tile_row(int t, int T) {
     return EX || t * 32 + 32 <= T ? t * 32 : T - 32;
 }
 
+// The tiles that the rows from r0 see: keys of queries, queries of keys.
+struct Tiles {
+    int first, last;
+    __device__ __forceinline__ int waves() const { return last - first + 1 < kWaves ? last - first + 1 : kWaves; }
+};
+__device__ __forceinline__ Tiles key_tiles(int r0, int T, int window) {
+    return {window > 0 && r0 > window ? (r0 - window) / 32 : 0, (r0 + 31 < T ? r0 + 31 : T - 1) / 32};
+}
+__device__ __forceinline__ Tiles query_tiles(int r0, int T, int window) {
+    return {r0 / 32, (window > 0 && r0 + 31 + window < T ? r0 + 31 + window : T - 1) / 32};
+}
+
 // ============================ forward ============================
 template <bool EX, int HD>
 __device__ __forceinline__ void fwd_tiles(f32x16 (&o)[HD / 32], float& m, float& l, const Own& w, const Src& q,
@@ -309,10 +323,9 @@ __device__ __forceinline__ void fwd_tiles(f32x16 (&o)[HD / 32], float& m, float&
     l = 0.f;
     const int qw = w.row0, my_q = qw + (lane & 31);
     if (qw >= T) return;
-    const int first = window > 0 && qw > window ? (qw - window) / 32 : 0;
-    const int last = (qw + 31 < T ? qw + 31 : T - 1) / 32;
+    const Tiles tiles = key_tiles(qw, T, window);
 #pragma unroll 1
-    for (int kt = first + kg; kt <= last; kt += kWaves) {
+    for (int kt = tiles.first + kg; kt <= tiles.last; kt += kWaves) {
         const int k0 = tile_row<EX>(kt, T);
         f32x16 s = row_products<EX, HD>(k, k0, T, w, q, lane);
         float mt = -INFINITY;
@@ -363,6 +376,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_k(float* out, float* lse
     const int64_t rs = (int64_t)H * HD, off = (int64_t)b * T * rs + (int64_t)h * HD;
     const Src q(qp + off, rs, lane), k(kp + off, rs, lane), v(vp + off, rs, lane);
     const Own w{smem, q0};
+    const int ng = key_tiles(q0, T, window).waves();
     const int valid = T - q0 < kRows ? T - q0 : kRows, my_q = w.row0 + lane;
 
     own_planes<HD>(smem, q, q0, T);
@@ -390,13 +404,13 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_k(float* out, float* lse
             const int i = g * 64 + (lane & 31);
             lt += ml[i + 32] * exp2_hw(ml[i] - m_use);
         }
-        put_block<HD>(regs + kg * kRows * ld_out<HD>(), o, exp2_hw(m - m_use), lane);
+        if (kg < ng) put_block<HD>(regs + kg * kRows * ld_out<HD>(), o, exp2_hw(m - m_use), lane);
         if (kg == 0 && lane < 32) {
             inv[lane] = lt > 0.f ? 1.0f / lt : 0.f;
             my_lse = lt > 0.f ? (mt + log2f(lt)) * kLn2 : -INFINITY;
         }
         __syncthreads();
-        bool bad = sum_blocks<HD>(y, regs, inv, valid);
+        bool bad = sum_blocks<HD>(y, regs, inv, valid, ng);
         bad |= kg == 0 && lane < 32 && my_q < T && !(fabsf(my_lse) <= 3.402823466e38f);
         if (!__syncthreads_or(bad) || pass == 1) break;
     }
@@ -414,10 +428,9 @@ __device__ __forceinline__ void dq_tiles(f32x16 (&acc)[HD / 32], const Own& w, c
     const int qw = w.row0, my_q = qw + (lane & 31);
     if (qw >= T) return;
     const Own wd{w.planes + 3 * kRows * HD * 2, w.row0};  // Q planes, then dO planes
-    const int first = window > 0 && qw > window ? (qw - window) / 32 : 0;
-    const int last = (qw + 31 < T ? qw + 31 : T - 1) / 32;
+    const Tiles tiles = key_tiles(qw, T, window);
 #pragma unroll 1
-    for (int kt = first + kg; kt <= last; kt += kWaves) {
+    for (int kt = tiles.first + kg; kt <= tiles.last; kt += kWaves) {
         const int k0 = tile_row<EX>(kt, T);
         const f32x16 s = row_products<EX, HD>(k, k0, T, w, q, lane);
         f32x16 ds = row_products<EX, HD>(v, k0, T, wd, dout, lane);
@@ -445,6 +458,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_dq_k(float* dq, const float*
     const int64_t rs = (int64_t)H * HD, off = (int64_t)b * T * rs + (int64_t)h * HD;
     const Src q(qp + off, rs, lane), k(kp + off, rs, lane), v(vp + off, rs, lane), dout(dop + off, rs, lane);
     const Own w{smem, q0};
+    const int ng = key_tiles(q0, T, window).waves();
     const int valid = T - q0 < kRows ? T - q0 : kRows, my_q = w.row0 + (lane & 31);
     const int64_t bth = ((int64_t)b * T + (my_q < T ? my_q : 0)) * H + h;
     const float lse2 = lse[bth] * kLog2e, dd = dbuf[bth];
@@ -460,9 +474,9 @@ __global__ __launch_bounds__(kThreads, 2) void attn_dq_k(float* dq, const float*
     for (int pass = T >= 32 ? 0 : 1;; ++pass) {
         if (pass == 1) dq_tiles<true, HD>(acc, w, q, k, v, dout, T, window, scale_log2, lse2, dd, kg, lane);
         __syncthreads();
-        put_block<HD>(regs + kg * kRows * ld_out<HD>(), acc, scale, lane);
+        if (kg < ng) put_block<HD>(regs + kg * kRows * ld_out<HD>(), acc, scale, lane);
         __syncthreads();
-        const bool bad = sum_blocks<HD>(y, regs, nullptr, valid);
+        const bool bad = sum_blocks<HD>(y, regs, nullptr, valid, ng);
         if (!__syncthreads_or(bad) || pass == 1) break;
     }
     store_blocks<HD>(dq + off + (int64_t)q0 * rs, rs, y, valid);
@@ -472,39 +486,50 @@ __global__ __launch_bounds__(kThreads, 2) void attn_dq_k(float* dq, const float*
 template <bool EX, int HD>
 __device__ __forceinline__ void dkv_tiles(f32x16 (&dka)[HD / 32], f32x16 (&dva)[HD / 32], const Own& w, const Src& q,
                                           const Src& k, const Src& v, const Src& dout, const float* lse,
-                                          const float* dbuf, int H, int T, int window, float scale_log2, int kg,
-                                          int lane) {
+                                          const float* dbuf, float* stat, int H, int T, int window,
+                                          float scale_log2, int kg, int lane) {
 #pragma unroll
     for (int dt = 0; dt < HD / 32; ++dt) dka[dt] = dva[dt] = zero16();
     const int kw = w.row0, my_k = kw + (lane & 31);
     if (kw >= T) return;
     const Own wv{w.planes + 3 * kRows * HD * 2, w.row0};  // K planes, then V planes
-    const int qlast = window > 0 && kw + 31 + window < T ? kw + 31 + window : T - 1;
+    const Tiles tiles = query_tiles(kw, T, window);
 #pragma unroll 1
-    for (int qt = kw / 32 + kg; qt <= qlast / 32; qt += kWaves) {
+    for (int qt = tiles.first + kg; qt <= tiles.last; qt += kWaves) {
         const int q0 = tile_row<EX>(qt, T);
+        // LSE and D of the tile's queries, a row per lane, on their way before the
+        // product that needs them, then from LDS.  (Loaded by the masked
+        // exponentials they were a chain of 16 trips to memory and 16 addresses in
+        // registers: B64 T128 H8 hd128 155 -> 105 us, hd64 60 -> 49.)
+        const int qr = q0 + (lane & 31);
+        const int64_t at = (int64_t)(!EX || qr < T ? qr : T - 1) * H;
+        if (lane < 32) {
+            stat[lane] = lse[at] * kLog2e;
+            stat[32 + lane] = dbuf[at];
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
         f32x16 p = row_products<EX, HD>(q, q0, T, w, k, lane);
-        float dd[16];
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
             const int qi = q0 + acc_row(e, lane);
             const bool ok = qi >= qt * 32 && my_k <= qi && qi < T && my_k < T && (window <= 0 || my_k >= qi - window);
-            const int64_t at = (int64_t)(!EX || qi < T ? qi : T - 1) * H;
-            dd[e] = dbuf[at];
-            p[e] = ok ? exp2_hw(p[e] * scale_log2 - lse[at] * kLog2e) : 0.f;
+            const float x = exp2_hw(p[e] * scale_log2 - stat[acc_row(e, lane)]);
+            p[e] = ok ? x : 0.f;
         }
         add_tile<EX, HD>(dva, dout, q0, T, p, lane);
         f32x16 ds = row_products<EX, HD>(dout, q0, T, wv, v, lane);
 #pragma unroll
-        for (int e = 0; e < 16; ++e) ds[e] = p[e] * (ds[e] - dd[e]);
+        for (int e = 0; e < 16; ++e) ds[e] = p[e] * (ds[e] - stat[32 + acc_row(e, lane)]);
         add_tile<EX, HD>(dka, q, q0, T, ds, lane);
     }
 }
 
 // OCC: workgroups per CU the registers allow.  At hd 128 one per CU (all of
 // both accumulators, both fragments and their loads in registers) is faster
-// while the grid gives each CU no more than two (B4 T512 H4: 41 against 54 us),
-// two with ~50 spilled registers beyond that (B16 T2048 H4: 1630 against 1900).
+// while each CU has no more than one (B4 T512 H4: 39 against 44 us), two with a
+// few spilled registers beyond that (B32 T64 H8: 34 against 39, B16 T2048 H4:
+// 1380 against 1720).
 template <int HD, int OCC>
 __global__ __launch_bounds__(kThreads, OCC) void attn_dkv_k(float* dk, float* dv, const float* qp, const float* kp,
                                                      const float* vp, const float* dop, const float* lse,
@@ -519,28 +544,30 @@ __global__ __launch_bounds__(kThreads, OCC) void attn_dkv_k(float* dk, float* dv
     const int64_t rs = (int64_t)H * HD, off = (int64_t)b * T * rs + (int64_t)h * HD;
     const Src q(qp + off, rs, lane), k(kp + off, rs, lane), v(vp + off, rs, lane), dout(dop + off, rs, lane);
     const Own w{smem, k0};
+    const int ng = query_tiles(k0, T, window).waves();
     const int valid = T - k0 < kRows ? T - k0 : kRows;
     const float* const lb = lse + (int64_t)b * T * H + h;
     const float* const db = dbuf + (int64_t)b * T * H + h;
+    float* const stat = reinterpret_cast<float*>(smem + attn_lds<HD, 2>() - kStatLds) + kg * 2 * kRows;
 
     own_planes<HD>(smem, k, k0, T);
     own_planes<HD>(smem + 3 * kRows * HD * 2, v, k0, T);
     __syncthreads();
     f32x16 dka[HD / 32], dva[HD / 32];
     if (T >= 32)
-        dkv_tiles<false, HD>(dka, dva, w, q, k, v, dout, lb, db, H, T, window, scale_log2, kg, lane);
+        dkv_tiles<false, HD>(dka, dva, w, q, k, v, dout, lb, db, stat, H, T, window, scale_log2, kg, lane);
     float4 yk[HD / 32], yv[HD / 32];
 #pragma unroll 1
     for (int pass = T >= 32 ? 0 : 1;; ++pass) {
-        if (pass == 1) dkv_tiles<true, HD>(dka, dva, w, q, k, v, dout, lb, db, H, T, window, scale_log2, kg, lane);
+        if (pass == 1) dkv_tiles<true, HD>(dka, dva, w, q, k, v, dout, lb, db, stat, H, T, window, scale_log2, kg, lane);
         __syncthreads();
-        put_block<HD>(regs + kg * kRows * ld_out<HD>(), dka, scale, lane);
+        if (kg < ng) put_block<HD>(regs + kg * kRows * ld_out<HD>(), dka, scale, lane);
         __syncthreads();
-        bool bad = sum_blocks<HD>(yk, regs, nullptr, valid);
+        bool bad = sum_blocks<HD>(yk, regs, nullptr, valid, ng);
         __syncthreads();
-        put_block<HD>(regs + kg * kRows * ld_out<HD>(), dva, 1.0f, lane);
+        if (kg < ng) put_block<HD>(regs + kg * kRows * ld_out<HD>(), dva, 1.0f, lane);
         __syncthreads();
-        bad |= sum_blocks<HD>(yv, regs, nullptr, valid);
+        bad |= sum_blocks<HD>(yv, regs, nullptr, valid, ng);
         if (!__syncthreads_or(bad) || pass == 1) break;
     }
     store_blocks<HD>(dk + off + (int64_t)k0 * rs, rs, yk, valid);
@@ -583,7 +610,7 @@ int32_t attn_launch(hipStream_t st, AttnOp op, float* o1, float* o2, const float
                                                             scale_log2, scale);                                      \
     } while (0)
     if constexpr (HD == 128) {
-        if (grid <= 512) AR_DKV(1);
+        if (grid <= 256) AR_DKV(1);
         else AR_DKV(2);
     } else {
         AR_DKV(2);
