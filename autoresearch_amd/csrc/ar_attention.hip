@@ -87,13 +87,14 @@ int32_t attn_padded(ar_stream_t stream, ar::AttnOp op, float* o1, float* o2, con
 }
 
 // One op with bf16 products on fp32 tensors, any head_dim: the two tensors
-// that several workgroups stream are rounded and padded into the workspace by
-// one launch, everything else is read and written where it is.  The workspace
-// is asked for every operand (and, padded, every result), as the op has
-// always documented.  Against a copy of each operand and of each padded
-// result, the four ops together: 708 -> 629 us at 16.8M values a tensor
-// (head_dim 128; 11 conversions of 18 us became three launches of 28), 189 ->
-// 134 us at a padded head_dim (96) and 1.7M.
+// that several workgroups stream (in short sequences all of them) are rounded
+// and padded into the workspace by one launch, everything else is read and
+// written where it is.  The workspace is asked for every operand (and, padded,
+// every result): what a call needs does not depend on the sequence's length.
+// Against a copy of each operand and of each padded result, the four ops
+// together: 708 -> 629 us at 16.8M values a tensor (head_dim 128; 11
+// conversions of 18 us became three launches of 28), 189 -> 134 us at a padded
+// head_dim (96) and 1.7M.
 int32_t attn_bf16(ar_stream_t stream, ar::AttnOp op, float* o1, float* o2, const float* const* in, const float* lse,
                   const float* dbuf, int64_t B, int64_t T, int64_t H, int64_t hd, int64_t window) {
     int32_t r = check_shape(B, T, H, hd);
@@ -106,8 +107,8 @@ int32_t attn_bf16(ar_stream_t stream, ar::AttnOp op, float* o1, float* o2, const
     int32_t st;
     char* w = (char*)ar::workspace(ar::S(stream), nin * each + nout * align256((size_t)n * sizeof(float)), &st);
     if (!w) return st;
-    return ar::flash_attn_f32(ar::S(stream), op, o1, o2, in[0], in[1], in[2], in[3], lse, dbuf, B, T, H, hd, window,
-                              (ar::bf16*)w, (ar::bf16*)(w + each));
+    return ar::flash_attn_f32(ar::S(stream), op, o1, o2, in, lse, dbuf, B, T, H, hd, window, (ar::bf16*)w,
+                              (int64_t)(each / sizeof(ar::bf16)));
 }
 }  // namespace
 

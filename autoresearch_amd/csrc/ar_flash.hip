@@ -1099,15 +1099,18 @@ int32_t flash_hd(hipStream_t st, AttnOp op, float* o1, float* o2, const FlashOut
     return check_launch("flash_attn_bwd_dkv (bf16 operands)");
 }
 
-// The streamed pair of an op on fp32 tensors: rows rounded to bf16 and
-// zero-padded from hd to HD columns, both tensors in one launch (blockIdx.y),
-// eight columns per thread.
+// Rounded copies of an op's fp32 tensors: rows rounded to bf16 and zero-padded
+// from hd to HD columns, all of them in one launch (blockIdx.y), eight columns
+// per thread.
+struct RoundSet {
+    const float* src[4];
+    bf16* dst[4];
+};
 template <int HD>
-__global__ __launch_bounds__(kThreads) void round_rows_k(bf16* d0, bf16* d1, const float* s0, const float* s1,
-                                                         int64_t rows, int hd) {
+__global__ __launch_bounds__(kThreads) void round_rows_k(RoundSet t, int64_t rows, int hd) {
     constexpr int CH = HD / 8;
-    bf16* const dst = blockIdx.y ? d1 : d0;
-    const float* const src = blockIdx.y ? s1 : s0;
+    bf16* const dst = t.dst[blockIdx.y];
+    const float* const src = t.src[blockIdx.y];
     for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < rows * CH; i += (int64_t)gridDim.x * kThreads) {
         const int64_t r = i / CH;
         const int c = (int)(i % CH) * 8;
@@ -1115,20 +1118,37 @@ __global__ __launch_bounds__(kThreads) void round_rows_k(bf16* d0, bf16* d1, con
     }
 }
 
+// in = {q, k, v, dO}.
 template <int HD>
-int32_t flash_f32_hd(hipStream_t st, AttnOp op, float* o1, float* o2, const float* q, const float* k, const float* v,
-                     const float* dout, const float* lse, const float* dbuf, int B, int T, int H, int hd, int window,
-                     bf16* w0, bf16* w1) {
+int32_t flash_f32_hd(hipStream_t st, AttnOp op, float* o1, float* o2, const float* const* in, const float* lse,
+                     const float* dbuf, int B, int T, int H, int hd, int window, bf16* w, int64_t wstep) {
     const float scale = 1.0f / sqrtf((float)hd);
     const float scale_log2 = scale * kLog2e;
     const unsigned grid = (unsigned)(((T + kOwn - 1) / kOwn) * B * H);
     const int64_t rs = (int64_t)H * hd, rows = (int64_t)B * T * H;
     const RowOut out1{o1, nullptr, rs, rs, nullptr, nullptr, 0, 1}, out2{o2, nullptr, rs, rs, nullptr, nullptr, 0, 1};
-    const dim3 rgrid(flat_grid(rows * (HD / 8), kThreads), 2);
-    if (op == AttnOp::DKV)
-        round_rows_k<HD><<<rgrid, kThreads, 0, st>>>(w0, w1, q, dout, rows, hd);
-    else
-        round_rows_k<HD><<<rgrid, kThreads, 0, st>>>(w0, w1, k, v, rows, hd);
+    // A sequence of one row block: its own rows are no fewer than what it
+    // streams, and read from fp32 a fragment takes 32 bytes of each of 32 rows,
+    // which evict each other from L1 where they lie a power of two apart.  So all
+    // operands are rounded (us, against own rows from fp32): forward B512 T32 H16
+    // hd128 255 -> 201, dK/dV B64 T128 H8 hd128 67 -> 54, B32 T33 H8 19 -> 16.
+    // Two row blocks already win by the other way (B32 T256 H8 66 either way).
+    const bool all = hd == HD && T <= kOwn;
+    RoundSet t{};
+    int n = 0;
+    for (int i = 0; i < (op == AttnOp::FWD ? 3 : 4); ++i) {
+        const bool streamed = op == AttnOp::DKV ? i == 0 || i == 3 : i == 1 || i == 2;
+        if (!all && !streamed) continue;
+        t.src[n] = in[i];
+        t.dst[n] = w + n * wstep;
+        ++n;
+    }
+    const dim3 rgrid(flat_grid(rows * (HD / 8), kThreads), n);
+    round_rows_k<HD><<<rgrid, kThreads, 0, st>>>(t, rows, hd);
+    if (all)
+        return flash_hd<HD>(st, op, o1, o2, FlashOut{}, t.dst[0], t.dst[1], t.dst[2], t.dst[3], lse, dbuf, B, T, H, window);
+    const float *q = in[0], *k = in[1], *v = in[2], *dout = in[3];
+    bf16 *const w0 = t.dst[0], *const w1 = t.dst[1];
     if (op == AttnOp::FWD)
         fa2_fwd_k<HD, float><<<grid, kThreads, fa2_lds<HD>(false), st>>>(out1, o2, q, w0, w1, B, T, H, window,
                                                                          scale_log2, hd);
@@ -1203,16 +1223,16 @@ int32_t flash_attn_bf16(hipStream_t st, AttnOp op, float* o1, float* o2, const F
     }
 }
 
-int32_t flash_attn_f32(hipStream_t st, AttnOp op, float* o1, float* o2, const float* q, const float* k,
-                       const float* v, const float* dout, const float* lse, const float* dbuf, int64_t B, int64_t T,
-                       int64_t H, int64_t hd, int64_t window, bf16* w0, bf16* w1) {
+int32_t flash_attn_f32(hipStream_t st, AttnOp op, float* o1, float* o2, const float* const* in, const float* lse,
+                       const float* dbuf, int64_t B, int64_t T, int64_t H, int64_t hd, int64_t window, bf16* w,
+                       int64_t wstep) {
     if (((T + kOwn - 1) / kOwn) * B * H > 0x7fffffff || T > (1 << 30))
         return set_error(AR_EINVAL, "flash attention: shape too large");
-    const int w = window > T ? (int)T : (int)window;
+    const int wd = window > T ? (int)T : (int)window;
     const int b = (int)B, t = (int)T, h = (int)H, d = (int)hd;
-    if (hd <= 32) return flash_f32_hd<32>(st, op, o1, o2, q, k, v, dout, lse, dbuf, b, t, h, d, w, w0, w1);
-    if (hd <= 64) return flash_f32_hd<64>(st, op, o1, o2, q, k, v, dout, lse, dbuf, b, t, h, d, w, w0, w1);
-    return flash_f32_hd<128>(st, op, o1, o2, q, k, v, dout, lse, dbuf, b, t, h, d, w, w0, w1);
+    if (hd <= 32) return flash_f32_hd<32>(st, op, o1, o2, in, lse, dbuf, b, t, h, d, wd, w, wstep);
+    if (hd <= 64) return flash_f32_hd<64>(st, op, o1, o2, in, lse, dbuf, b, t, h, d, wd, w, wstep);
+    return flash_f32_hd<128>(st, op, o1, o2, in, lse, dbuf, b, t, h, d, wd, w, wstep);
 }
 
 }  // namespace ar

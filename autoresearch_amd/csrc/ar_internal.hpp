@@ -131,12 +131,13 @@ struct FlashOut {
 int32_t flash_attn_bf16(hipStream_t st, AttnOp op, float* o1, float* o2, const FlashOut& fo, const bf16* q,
                         const bf16* k, const bf16* v, const bf16* dout, const float* lse, const float* dbuf, int64_t B,
                         int64_t T, int64_t H, int64_t HD, int64_t window);
-// The same products from fp32 tensors of any head_dim hd in [1, 128], rounded
-// to bf16 as they are read; w0, w1 hold the rounded copies of the two tensors
-// that several workgroups read (B T H rows of hd's next size of 32, 64, 128).
-int32_t flash_attn_f32(hipStream_t st, AttnOp op, float* o1, float* o2, const float* q, const float* k,
-                       const float* v, const float* dout, const float* lse, const float* dbuf, int64_t B, int64_t T,
-                       int64_t H, int64_t hd, int64_t window, bf16* w0, bf16* w1);
+// The same products from fp32 tensors in = {q, k, v, dO} of any head_dim hd in
+// [1, 128], rounded to bf16 as they are read; w holds the rounded copies, wstep
+// elements apart, of the tensors that several workgroups read, or of all of
+// them (B T H rows of hd's next size of 32, 64, 128 each).
+int32_t flash_attn_f32(hipStream_t st, AttnOp op, float* o1, float* o2, const float* const* in, const float* lse,
+                       const float* dbuf, int64_t B, int64_t T, int64_t H, int64_t hd, int64_t window, bf16* w,
+                       int64_t wstep);
 // dS workspace size (bf16 elements) of a DKV launch with FlashOut::ds.
 int64_t flash_ds_elems(int64_t B, int64_t T, int64_t H);
 // D = rowsum(dO * O) per (token, head) from bf16 dO [B, T, H, hd] and fp32 O.

@@ -12,7 +12,9 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("B,T,H,hd,window", [
     (1, 33, 2, 32, 0), (2, 129, 3, 64, 0), (1, 300, 2, 128, 70), (1, 64, 2, 1, 0), (1, 65, 3, 5, 16), (2, 127, 1, 30, 0),
     (1, 128, 2, 33, 0), (1, 200, 2, 50, 64), (2, 257, 2, 63, 0), (1, 161, 3, 80, 100), (2, 31, 1, 97, 0),
-    (1, 260, 2, 126, 0), (1, 5, 1, 127, 2), (1, 1, 1, 48, 0)])
+    (1, 260, 2, 126, 0), (1, 5, 1, 127, 2), (1, 1, 1, 48, 0),
+    # one 128-row block of a tiled size: every operand is rounded
+    (2, 128, 3, 128, 0), (3, 100, 2, 64, 40), (2, 1, 2, 32, 0)])
 def test_bf16_attention_of_fp32_tensors_vs_fp64(B, T, H, hd, window):
     import torch
     from autoresearch_amd import ops
