@@ -29,9 +29,21 @@
 // Nothing is staged and there is no barrier in the tile loop.
 //
 // The small terms of a product have their own accumulator, added to the large
-// one per tile.  A block whose result is not finite, or holds values below
-// 2^-100, is formed again on the fp32 matrix cores (EX), so infinities, NaN and
-// magnitudes that bf16 has no low bits for give what fp32 products give.
+// one per tile.
+//
+// Magnitudes.  The split is exact for zero and from 2^-110 to 3.39e38; below, a
+// value loses up to 2^-134, and a block where that could show is formed on the
+// fp32 matrix cores (EX):
+//   * an own row with such a value;
+//   * a result that is not finite (infinities, NaN, what bf16 rounds to infinity);
+//   * a result below kSmall, or a magnitude above kBig among the own rows, the
+//     streamed rows that form S and the dS, if the streamed rows hold a value
+//     below 2^-110.
+// Otherwise what is lost is below fp32's own rounding.  hd 2^-134 kBig = 2^-109
+// of a score or of dP changes no exponential and moves a result by 2^-109 kBig
+// per unit of P, the T 2^-134 kBig of small dS less; O and dV, formed from P
+// 2^24 (so P keeps every bit above 2^-126), by 2^-134 per unit of P.  Against
+// 2^-24 kSmall that leaves T up to 2^17.
 //
 // dK/dV are accumulated by key ownership and dQ by query ownership (no
 // atomics: deterministic).
@@ -43,6 +55,7 @@ namespace {
 
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLn2 = 0.6931471805599453f;
+constexpr float kTiny = 0x1p-110f, kBig = 0x1p18f, kSmall = 0x1p-48f, kScaleP = 0x1p24f;
 constexpr int kRows = 32, kWaves = 4, kThreads = kWaves * kWave;  // own rows and waves of a workgroup
 
 __device__ __forceinline__ int acc_row(int v, int lane) { return (v >> 2) * 8 + (lane >> 5) * 4 + (v & 3); }
@@ -136,20 +149,48 @@ __device__ __forceinline__ void col_vals(float (&x)[8], const Src& t, int row0, 
         }
     }
 }
-__device__ __forceinline__ void acc_vals(float (&x)[8], const f32x16& a, int s) {
+__device__ __forceinline__ void acc_vals(float (&x)[8], const f32x16& a, int s, float f) {
 #pragma unroll
-    for (int e = 0; e < 8; ++e) x[e] = a[8 * s + e];
+    for (int e = 0; e < 8; ++e) x[e] = a[8 * s + e] * f;
+}
+
+// What a thread has met: its least magnitude that is not zero and its largest.
+struct Range {
+    unsigned least = ~0u;  // twice the bits, less one: zero of either sign wraps to the top
+    float most = 0.f;
+    __device__ __forceinline__ void see(float x) {
+        const unsigned u = __float_as_uint(x) * 2u - 1u;
+        least = u < least ? u : least;
+        most = fmaxf(most, fabsf(x));
+    }
+    __device__ __forceinline__ bool tiny() const { return least < __float_as_uint(kTiny) * 2u - 1u; }
+    __device__ __forceinline__ bool big() const { return most > kBig; }
+};
+// Whether rows [r0, r1) hold a value below kTiny that is not zero, asked by the whole workgroup.
+template <int HD>
+__device__ __forceinline__ bool rows_tiny(const Src& t, int r0, int r1) {
+    Range f;
+#pragma unroll 2
+    for (int r = r0 + (int)threadIdx.x / (HD / 8); r < r1; r += kThreads / (HD / 8)) {
+        float x[8];
+        ld8(x, t.base + (int64_t)r * t.rs + threadIdx.x % (HD / 8) * 8);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) f.see(x[e]);
+    }
+    return f.tiny();
 }
 
 // Split planes of the own rows of an operand in LDS (K-major units, kslot
 // order), written by the whole workgroup.
 template <int HD>
-__device__ __forceinline__ void own_planes(unsigned char* planes, const Src& t, int row0, int T) {
+__device__ __forceinline__ void own_planes(unsigned char* planes, const Src& t, int row0, int T, Range& seen) {
     constexpr int U = HD / 8, PB = kRows * HD * 2;
     for (int it = threadIdx.x; it < kRows * U; it += kThreads) {
         const int r = it / U, c = it % U, row = row0 + r;
         float x[8];
         ld8(x, t.base + (int64_t)(row < T ? row : T - 1) * t.rs + c * 8);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) seen.see(x[e]);
         const Frag<false> f(x);
         const int o = kslot<U>(r, c) * 16;
 #pragma unroll
@@ -173,14 +214,15 @@ __device__ __forceinline__ Frag<EX> own_frag(const Own& w, const Src& t, int T, 
     }
 }
 
-// c[cols] += X^T . B for the 32-row tile of X at row0 (columns dt 32..) and the
-// 32 x 32 block b (accumulator layout): the small terms of the tile are summed apart.
+// c[cols] += X^T . (f B) for the 32-row tile of X at row0 (columns dt 32..) and
+// the 32 x 32 block b (accumulator layout): the small terms of the tile are
+// summed apart.
 template <bool EX, int HD>
-__device__ __forceinline__ void add_tile(f32x16 (&c)[HD / 32], const Src& t, int row0, int T, const f32x16& b, int lane) {
+__device__ __forceinline__ void add_tile(f32x16 (&c)[HD / 32], const Src& t, int row0, int T, const f32x16& b, float f, int lane) {
     float x[8];
-    acc_vals(x, b, 0);
+    acc_vals(x, b, 0, f);
     const Frag<EX> b0(x);
-    acc_vals(x, b, 1);
+    acc_vals(x, b, 1, f);
     const Frag<EX> b1(x);
 #pragma unroll
     for (int dt = 0; dt < HD / 32; ++dt) {
@@ -196,14 +238,20 @@ __device__ __forceinline__ void add_tile(f32x16 (&c)[HD / 32], const Src& t, int
     }
 }
 
-// The 32 x 32 block of (streamed rows at row0) . (own rows)^T.
+// The 32 x 32 block of (streamed rows at row0) . (own rows)^T.  most: the largest
+// streamed magnitude so far (null: not asked for).
 template <bool EX, int HD>
-__device__ __forceinline__ f32x16 row_products(const Src& t, int row0, int T, const Own& w, const Src& own, int lane) {
+__device__ __forceinline__ f32x16 row_products(const Src& t, int row0, int T, const Own& w, const Src& own, int lane,
+                                               float* most = nullptr) {
     f32x16 c = zero16(), low = zero16();
 #pragma unroll
     for (int ks = 0; ks < HD / 16; ++ks) {
         float x[8];
         row_vals<EX>(x, t, row0, T, ks, lane);
+        if (!EX && most) {
+#pragma unroll
+            for (int e = 0; e < 8; e += 2) *most = fmaxf(fmaxf(fabsf(x[e]), fabsf(x[e + 1])), *most);
+        }
         dot16(c, low, Frag<EX>(x), own_frag<EX, HD>(w, own, T, ks, lane));
         // two k-steps' loads in flight: with all HD / 16 hoisted dQ spills at hd
         // 128 and every kernel was slower (B16 T2048: fwd 552 -> 530 us, dQ 896 -> 842)
@@ -247,13 +295,12 @@ __device__ __forceinline__ void put_block(float* reg, const f32x16 (&acc)[HD / 3
 }
 
 // Sums the regions of each row over the first ng waves (those that had a tile),
-// in order, times scale_row[row]; y holds this thread's float4s.  Returns whether one of a valid row is not finite or
-// below 2^-100.
+// in order, times scale_row[row]; y holds this thread's float4s.  inf, small:
+// whether one of a valid row is not finite / below kSmall.
 template <int HD>
-__device__ __forceinline__ bool sum_blocks(float4 (&y)[HD / 32], const float* regs, const float* scale_row,
-                                           int valid, int ng) {
+__device__ __forceinline__ void sum_blocks(float4 (&y)[HD / 32], const float* regs, const float* scale_row,
+                                           int valid, int ng, bool& inf, bool& small) {
     constexpr int RB = kRows * ld_out<HD>();
-    bool bad = false;
 #pragma unroll
     for (int n = 0; n < HD / 32; ++n) {
         const int i = (n * kThreads + (int)threadIdx.x) * 4, r = i / HD, d = i % HD;
@@ -268,11 +315,10 @@ __device__ __forceinline__ bool sum_blocks(float4 (&y)[HD / 32], const float* re
         const float f = scale_row ? scale_row[r] : 1.0f;
         t = make_float4(t.x * f, t.y * f, t.z * f, t.w * f);
         y[n] = t;
-        const float m = fmaxf(fmaxf(fabsf(t.x), fabsf(t.y)), fmaxf(fabsf(t.z), fabsf(t.w)));
         const bool fine = (t.x - t.x) + (t.y - t.y) + (t.z - t.z) + (t.w - t.w) == 0.f;
-        bad |= r < valid && (!fine || (m > 0.f && m < 7.8886e-31f));
+        inf |= r < valid && !fine;
+        small |= r < valid && fminf(fminf(fabsf(t.x), fabsf(t.y)), fminf(fabsf(t.z), fabsf(t.w))) < kSmall;
     }
-    return bad;
 }
 template <int HD>
 __device__ __forceinline__ void store_blocks(float* out, int64_t rs, const float4 (&y)[HD / 32], int valid) {
@@ -356,12 +402,12 @@ __device__ __forceinline__ void fwd_tiles(f32x16 (&o)[HD / 32], float& m, float&
                 for (int e = 0; e < 16; ++e) o[dt][e] *= alpha;
         }
         m = m_new;
-        add_tile<EX, HD>(o, v, k0, T, s, lane);
+        add_tile<EX, HD>(o, v, k0, T, s, EX ? 1.f : kScaleP, lane);
     }
 }
 
 template <int HD>
-__global__ __launch_bounds__(kThreads, 2) void attn_fwd_k(float* out, float* lse, const float* qp, const float* kp,
+__global__ __launch_bounds__(kThreads, HD == 128 ? 2 : HD == 64 ? 3 : 4) void attn_fwd_k(float* out, float* lse, const float* qp, const float* kp,
                                                      const float* vp, int T, int H, int nblk, int heads, int window,
                                                      float scale_log2) {
     extern __shared__ __align__(16) unsigned char smem[];
@@ -376,10 +422,12 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_k(float* out, float* lse
     const int64_t rs = (int64_t)H * HD, off = (int64_t)b * T * rs + (int64_t)h * HD;
     const Src q(qp + off, rs, lane), k(kp + off, rs, lane), v(vp + off, rs, lane);
     const Own w{smem, q0};
-    const int ng = key_tiles(q0, T, window).waves();
+    const Tiles seen = key_tiles(q0, T, window);
+    const int ng = seen.waves();
     const int valid = T - q0 < kRows ? T - q0 : kRows, my_q = w.row0 + lane;
 
-    own_planes<HD>(smem, q, q0, T);
+    Range mine;
+    own_planes<HD>(smem, q, q0, T, mine);
     __syncthreads();
     f32x16 o[HD / 32];
     float m, l;
@@ -406,13 +454,16 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_k(float* out, float* lse
         }
         if (kg < ng) put_block<HD>(regs + kg * kRows * ld_out<HD>(), o, exp2_hw(m - m_use), lane);
         if (kg == 0 && lane < 32) {
-            inv[lane] = lt > 0.f ? 1.0f / lt : 0.f;
+            inv[lane] = lt > 0.f ? (pass == 0 ? 1.0f / kScaleP : 1.0f) / lt : 0.f;
             my_lse = lt > 0.f ? (mt + log2f(lt)) * kLn2 : -INFINITY;
         }
         __syncthreads();
-        bool bad = sum_blocks<HD>(y, regs, inv, valid, ng);
-        bad |= kg == 0 && lane < 32 && my_q < T && !(fabsf(my_lse) <= 3.402823466e38f);
-        if (!__syncthreads_or(bad) || pass == 1) break;
+        bool redo = mine.tiny() || (kg == 0 && lane < 32 && my_q < T && !(fabsf(my_lse) <= 3.402823466e38f));
+        bool look = mine.big();
+        sum_blocks<HD>(y, regs, inv, valid, ng, redo, look);
+        if (pass == 1 || !__syncthreads_or(redo || look)) break;
+        const int r0 = seen.first * 32, r1 = q0 + valid;
+        if (!__syncthreads_or(redo) && !__syncthreads_or(rows_tiny<HD>(k, r0, r1) || rows_tiny<HD>(v, r0, r1))) break;
     }
     store_blocks<HD>(out + off + (int64_t)q0 * rs, rs, y, valid);
     if (kg == 0 && lane < 32 && my_q < T) lse[((int64_t)b * T + my_q) * H + h] = my_lse;
@@ -422,7 +473,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_k(float* out, float* lse
 template <bool EX, int HD>
 __device__ __forceinline__ void dq_tiles(f32x16 (&acc)[HD / 32], const Own& w, const Src& q, const Src& k, const Src& v,
                                          const Src& dout, int T, int window, float scale_log2, float lse2, float dd,
-                                         int kg, int lane) {
+                                         float& most, int kg, int lane) {
 #pragma unroll
     for (int dt = 0; dt < HD / 32; ++dt) acc[dt] = zero16();
     const int qw = w.row0, my_q = qw + (lane & 31);
@@ -432,7 +483,7 @@ __device__ __forceinline__ void dq_tiles(f32x16 (&acc)[HD / 32], const Own& w, c
 #pragma unroll 1
     for (int kt = tiles.first + kg; kt <= tiles.last; kt += kWaves) {
         const int k0 = tile_row<EX>(kt, T);
-        const f32x16 s = row_products<EX, HD>(k, k0, T, w, q, lane);
+        const f32x16 s = row_products<EX, HD>(k, k0, T, w, q, lane, &most);
         f32x16 ds = row_products<EX, HD>(v, k0, T, wd, dout, lane);
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
@@ -440,13 +491,14 @@ __device__ __forceinline__ void dq_tiles(f32x16 (&acc)[HD / 32], const Own& w, c
             const bool ok = key >= kt * 32 && key <= my_q && key < T && my_q < T && (window <= 0 || key >= my_q - window);
             const float p = ok ? exp2_hw(s[e] * scale_log2 - lse2) : 0.f;
             ds[e] = p * (ds[e] - dd);
+            if (!EX) most = fmaxf(most, fabsf(ds[e]));
         }
-        add_tile<EX, HD>(acc, k, k0, T, ds, lane);
+        add_tile<EX, HD>(acc, k, k0, T, ds, 1.f, lane);
     }
 }
 
 template <int HD>
-__global__ __launch_bounds__(kThreads, 2) void attn_dq_k(float* dq, const float* qp, const float* kp, const float* vp,
+__global__ __launch_bounds__(kThreads, HD == 128 ? 2 : HD == 64 ? 3 : 4) void attn_dq_k(float* dq, const float* qp, const float* kp, const float* vp,
                                                     const float* dop, const float* lse, const float* dbuf, int T, int H,
                                                     int nblk, int heads, int window, float scale_log2, float scale) {
     extern __shared__ __align__(16) unsigned char smem[];
@@ -458,26 +510,31 @@ __global__ __launch_bounds__(kThreads, 2) void attn_dq_k(float* dq, const float*
     const int64_t rs = (int64_t)H * HD, off = (int64_t)b * T * rs + (int64_t)h * HD;
     const Src q(qp + off, rs, lane), k(kp + off, rs, lane), v(vp + off, rs, lane), dout(dop + off, rs, lane);
     const Own w{smem, q0};
-    const int ng = key_tiles(q0, T, window).waves();
+    const Tiles seen = key_tiles(q0, T, window);
+    const int ng = seen.waves();
     const int valid = T - q0 < kRows ? T - q0 : kRows, my_q = w.row0 + (lane & 31);
     const int64_t bth = ((int64_t)b * T + (my_q < T ? my_q : 0)) * H + h;
     const float lse2 = lse[bth] * kLog2e, dd = dbuf[bth];
 
-    own_planes<HD>(smem, q, q0, T);
-    own_planes<HD>(smem + 3 * kRows * HD * 2, dout, q0, T);
+    Range mine;
+    own_planes<HD>(smem, q, q0, T, mine);
+    own_planes<HD>(smem + 3 * kRows * HD * 2, dout, q0, T, mine);
     __syncthreads();
     f32x16 acc[HD / 32];
-    if (T >= 32)
-        dq_tiles<false, HD>(acc, w, q, k, v, dout, T, window, scale_log2, lse2, dd, kg, lane);
+    float most = 0.f;
+    if (T >= 32) dq_tiles<false, HD>(acc, w, q, k, v, dout, T, window, scale_log2, lse2, dd, most, kg, lane);
     float4 y[HD / 32];
 #pragma unroll 1
     for (int pass = T >= 32 ? 0 : 1;; ++pass) {
-        if (pass == 1) dq_tiles<true, HD>(acc, w, q, k, v, dout, T, window, scale_log2, lse2, dd, kg, lane);
+        if (pass == 1) dq_tiles<true, HD>(acc, w, q, k, v, dout, T, window, scale_log2, lse2, dd, most, kg, lane);
         __syncthreads();
         if (kg < ng) put_block<HD>(regs + kg * kRows * ld_out<HD>(), acc, scale, lane);
         __syncthreads();
-        const bool bad = sum_blocks<HD>(y, regs, nullptr, valid, ng);
-        if (!__syncthreads_or(bad) || pass == 1) break;
+        bool redo = mine.tiny(), look = mine.big() || most > kBig;
+        sum_blocks<HD>(y, regs, nullptr, valid, ng, redo, look);
+        if (pass == 1 || !__syncthreads_or(redo || look)) break;
+        const int r0 = seen.first * 32, r1 = q0 + valid;
+        if (!__syncthreads_or(redo) && !__syncthreads_or(rows_tiny<HD>(k, r0, r1) || rows_tiny<HD>(v, r0, r1))) break;
     }
     store_blocks<HD>(dq + off + (int64_t)q0 * rs, rs, y, valid);
 }
@@ -487,7 +544,7 @@ template <bool EX, int HD>
 __device__ __forceinline__ void dkv_tiles(f32x16 (&dka)[HD / 32], f32x16 (&dva)[HD / 32], const Own& w, const Src& q,
                                           const Src& k, const Src& v, const Src& dout, const float* lse,
                                           const float* dbuf, float* stat, int H, int T, int window,
-                                          float scale_log2, int kg, int lane) {
+                                          float scale_log2, float& most, int kg, int lane) {
 #pragma unroll
     for (int dt = 0; dt < HD / 32; ++dt) dka[dt] = dva[dt] = zero16();
     const int kw = w.row0, my_k = kw + (lane & 31);
@@ -509,7 +566,7 @@ __device__ __forceinline__ void dkv_tiles(f32x16 (&dka)[HD / 32], f32x16 (&dva)[
         }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
-        f32x16 p = row_products<EX, HD>(q, q0, T, w, k, lane);
+        f32x16 p = row_products<EX, HD>(q, q0, T, w, k, lane, &most);
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
             const int qi = q0 + acc_row(e, lane);
@@ -517,11 +574,14 @@ __device__ __forceinline__ void dkv_tiles(f32x16 (&dka)[HD / 32], f32x16 (&dva)[
             const float x = exp2_hw(p[e] * scale_log2 - stat[acc_row(e, lane)]);
             p[e] = ok ? x : 0.f;
         }
-        add_tile<EX, HD>(dva, dout, q0, T, p, lane);
+        add_tile<EX, HD>(dva, dout, q0, T, p, EX ? 1.f : kScaleP, lane);
         f32x16 ds = row_products<EX, HD>(dout, q0, T, wv, v, lane);
 #pragma unroll
-        for (int e = 0; e < 16; ++e) ds[e] = p[e] * (ds[e] - stat[32 + acc_row(e, lane)]);
-        add_tile<EX, HD>(dka, q, q0, T, ds, lane);
+        for (int e = 0; e < 16; ++e) {
+            ds[e] = p[e] * (ds[e] - stat[32 + acc_row(e, lane)]);
+            if (!EX) most = fmaxf(most, fabsf(ds[e]));
+        }
+        add_tile<EX, HD>(dka, q, q0, T, ds, 1.f, lane);
     }
 }
 
@@ -544,31 +604,37 @@ __global__ __launch_bounds__(kThreads, OCC) void attn_dkv_k(float* dk, float* dv
     const int64_t rs = (int64_t)H * HD, off = (int64_t)b * T * rs + (int64_t)h * HD;
     const Src q(qp + off, rs, lane), k(kp + off, rs, lane), v(vp + off, rs, lane), dout(dop + off, rs, lane);
     const Own w{smem, k0};
-    const int ng = query_tiles(k0, T, window).waves();
+    const Tiles seen = query_tiles(k0, T, window);
+    const int ng = seen.waves();
     const int valid = T - k0 < kRows ? T - k0 : kRows;
     const float* const lb = lse + (int64_t)b * T * H + h;
     const float* const db = dbuf + (int64_t)b * T * H + h;
     float* const stat = reinterpret_cast<float*>(smem + attn_lds<HD, 2>() - kStatLds) + kg * 2 * kRows;
 
-    own_planes<HD>(smem, k, k0, T);
-    own_planes<HD>(smem + 3 * kRows * HD * 2, v, k0, T);
+    Range mine;
+    own_planes<HD>(smem, k, k0, T, mine);
+    own_planes<HD>(smem + 3 * kRows * HD * 2, v, k0, T, mine);
     __syncthreads();
     f32x16 dka[HD / 32], dva[HD / 32];
-    if (T >= 32)
-        dkv_tiles<false, HD>(dka, dva, w, q, k, v, dout, lb, db, stat, H, T, window, scale_log2, kg, lane);
+    float most = 0.f;
+    if (T >= 32) dkv_tiles<false, HD>(dka, dva, w, q, k, v, dout, lb, db, stat, H, T, window, scale_log2, most, kg, lane);
     float4 yk[HD / 32], yv[HD / 32];
 #pragma unroll 1
     for (int pass = T >= 32 ? 0 : 1;; ++pass) {
-        if (pass == 1) dkv_tiles<true, HD>(dka, dva, w, q, k, v, dout, lb, db, stat, H, T, window, scale_log2, kg, lane);
+        if (pass == 1)
+            dkv_tiles<true, HD>(dka, dva, w, q, k, v, dout, lb, db, stat, H, T, window, scale_log2, most, kg, lane);
         __syncthreads();
         if (kg < ng) put_block<HD>(regs + kg * kRows * ld_out<HD>(), dka, scale, lane);
         __syncthreads();
-        bool bad = sum_blocks<HD>(yk, regs, nullptr, valid, ng);
+        bool redo = mine.tiny(), look = mine.big() || most > kBig;
+        sum_blocks<HD>(yk, regs, nullptr, valid, ng, redo, look);
         __syncthreads();
-        if (kg < ng) put_block<HD>(regs + kg * kRows * ld_out<HD>(), dva, 1.0f, lane);
+        if (kg < ng) put_block<HD>(regs + kg * kRows * ld_out<HD>(), dva, pass == 0 ? 1.0f / kScaleP : 1.0f, lane);
         __syncthreads();
-        bad |= sum_blocks<HD>(yv, regs, nullptr, valid, ng);
-        if (!__syncthreads_or(bad) || pass == 1) break;
+        sum_blocks<HD>(yv, regs, nullptr, valid, ng, redo, look);
+        if (pass == 1 || !__syncthreads_or(redo || look)) break;
+        const int r1 = seen.last * 32 + 32 < T ? seen.last * 32 + 32 : T;
+        if (!__syncthreads_or(redo) && !__syncthreads_or(rows_tiny<HD>(q, k0, r1) || rows_tiny<HD>(dout, k0, r1))) break;
     }
     store_blocks<HD>(dk + off + (int64_t)k0 * rs, rs, yk, valid);
     store_blocks<HD>(dv + off + (int64_t)k0 * rs, rs, yv, valid);
@@ -613,7 +679,7 @@ int32_t attn_launch(hipStream_t st, AttnOp op, float* o1, float* o2, const float
         if (grid <= 256) AR_DKV(1);
         else AR_DKV(2);
     } else {
-        AR_DKV(2);
+        AR_DKV(HD == 64 ? 2 : 3);
     }
 #undef AR_DKV
     return check_launch("flash_attn_bwd_dkv");

@@ -91,4 +91,69 @@ def test_fp32_attention_non_finite_and_tiny(env, T):
         assert float((o[b].double() - ref[0][b]).norm() / ref[0][b].norm()) <= 1e-6
     assert float((lse.double() - ref[1]).norm() / ref[1].norm()) <= 1e-6
     for a, b in zip((dq, dk, dv), ref[2:]):
-        assert float((a[2].double() - b[2]).norm() / b[2].norm()) <= 1e-6
+        for i, h in ((2, slice(None)), (1, slice(None)), (0, slice(0, 1))):  # untouched, tiny, the infinity's neighbour
+            x, y = a[i, :, h].double(), b[i, :, h]
+            assert float((x - y).norm() / y.norm()) <= 1e-6
+
+
+def _close(torch, got, ref, tol, dim):
+    err, size = (got.double() - ref).norm(dim=dim), ref.norm(dim=dim)
+    assert bool(torch.isfinite(got).all())
+    assert bool((err <= tol * size).all()), float((err / size.clamp_min(1e-300)).max())
+
+
+# powers of two on q, k, v, dO: values below 2^-110 of one operand behind
+# ordinary results (the other operand large), small results of ordinary
+# products, and the second pass of every kernel
+@pytest.mark.parametrize("sq,sk,sv,sdo", [(112, -112, 0, 0), (-112, 112, 0, 0), (0, 0, -116, 116), (0, 0, 100, -118),
+                                          (100, -100, 108, -112), (-100, 100, -116, 120), (-60, 60, -50, 60),
+                                          (0, 0, -112, 40), (0, 0, -109, 109), (0, 0, 0, -111)])
+@pytest.mark.parametrize("T,hd,window", [(40, 128, 0), (130, 64, 50), (257, 32, 0)])
+def test_fp32_attention_of_small_values(env, sq, sk, sv, sdo, T, hd, window):
+    """Scaling by powers of two is exact, so the results' relative errors are
+    those of test_fp32_attention_vs_fp64 (the terms of every result are 2^-118 or
+    more in size, so fp32's own subnormal roundings, 2^-149 each, do not show)."""
+    torch, ops = env
+    q, k, v, do = _inputs(torch, 2, T, 2, hd, T + hd)
+    q, k, v, do = q * 2.0 ** sq, k * 2.0 ** sk, v * 2.0 ** sv, do * 2.0 ** sdo
+    got, ref = _run(torch, ops, q, k, v, do, window), _exact(torch, q, k, v, do, window)
+    for name, a, b in zip(("o", "lse", "dq", "dk", "dv"), got, ref):
+        _close(torch, a, b, 2e-6, (1, 3) if name != "lse" else 1)
+
+
+@pytest.mark.parametrize("T", [40, 130])
+def test_fp32_attention_of_small_values_beside_large(env, T):
+    """Single columns below 2^-110 beside ordinary ones: every column of O, dK,
+    dV and dQ keeps fp32's accuracy by itself (column 3 of V and column 2 of Q,
+    K and dO are small, with dO's column 3 and one of q and k large)."""
+    torch, ops = env
+    q, k, v, do = _inputs(torch, 1, T, 2, 64, T)
+    v[..., 3] *= 2.0 ** -116
+    do[..., 3] *= 2.0 ** 20
+    k[..., 2] *= 2.0 ** -118
+    q[..., 2] *= 2.0 ** 30
+    do[..., 2] *= 2.0 ** -114
+    got, ref = _run(torch, ops, q, k, v, do, 0), _exact(torch, q, k, v, do, 0)
+    for a, b in zip((got[0],) + got[2:], (ref[0],) + ref[2:]):
+        _close(torch, a, b, 4e-6, 1)
+
+
+@pytest.mark.parametrize("T", [40, 130])
+def test_fp32_attention_second_pass_is_finite(env, T):
+    """A finite value that bf16 rounds to infinity has the blocks it reaches
+    formed again: their results, and those of the rows beside it, as fp64 has
+    them (dO's large value meets a column of V, and so of O, that is zero)."""
+    torch, ops = env
+    q, k, v, do = _inputs(torch, 2, T, 2, 128, T)
+    v[0, :, 1, 5] = 0.0
+    do[0, 20, 1, 5] = 3.3999e38
+    got, ref = _run(torch, ops, q, k, v, do, 0), _exact(torch, q, k, v, do, 0)
+    for a, b in zip(got[2:4], ref[2:4]):
+        _close(torch, a, b, 1e-6, (1, 3))
+    a, b = got[4], ref[4]
+    _close(torch, a[0, :, 1, 5][None, :21], b[0, :, 1, 5][None, :21], 1e-6, 1)
+    a[0, :, 1, 5] = b[0, :, 1, 5].float()  # (the keys after query 20 have the other queries' ordinary sums)
+    _close(torch, a, b, 1e-6, (1, 3))
+    v[0, 20, 1, 5] = 3.3999e38
+    o, lse = _run(torch, ops, q, k, v, do, 0)[:2]
+    _close(torch, o, _exact(torch, q, k, v, do, 0)[0], 1e-6, 1)
