@@ -747,10 +747,11 @@ struct X3Plan {
 // stage each) against the others' one (us, against L or M where it was chosen):
 //   8192 x 4096, C += :    R 16 86 -> 62   R 32 80 -> 51   R 64 88 -> 67   R 96 97 -> 81
 //   8192 x 4096, NT:       R 16 44 -> 38   R 32 42 -> 37   R 48 54 -> 50   (64: 51 -> 55)
-//   2048 x 1024, C += :    R 32 10 -> 8.4  R 96 13 -> 10   (100 with two stages: no gain)
-// With B MN-major and nothing to add, D and L are even.
+//   1024 x 512, C += / NT: R 16 9.9 -> 5.3 / 7.0 -> 4.4    512 x 512: 5.6 -> 5.1 / 4.8 -> 4.3
+// With B MN-major and nothing to add, D and L are even.  Below 48 blocks T's
+// shared reduction leaves more of the chip at work.
 X3Plan x3_plan(bool nt, int64_t M, int64_t N, int64_t K, int64_t batch, int64_t max_splits, bool aux) {
-    if (K <= (aux ? 96 : nt ? 48 : 0) && cdiv(M, X3D::BM) * cdiv(N, X3D::BN) * batch >= 256) return X3Plan{kX3D, 1};
+    if (K <= (aux ? 96 : nt ? 48 : 0) && cdiv(M, X3D::BM) * cdiv(N, X3D::BN) * batch >= 48) return X3Plan{kX3D, 1};
     X3Plan best{0, 1};
     double least = 1e30;
     for (int t = 0; t < kX3Tiles; ++t) {
