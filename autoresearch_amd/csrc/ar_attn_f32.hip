@@ -557,7 +557,7 @@ __device__ __forceinline__ void dkv_tiles(f32x16 (&dka)[HD / 32], f32x16 (&dva)[
         // LSE and D of the tile's queries, a row per lane, on their way before the
         // product that needs them, then from LDS.  (Loaded by the masked
         // exponentials they were a chain of 16 trips to memory and 16 addresses in
-        // registers: B64 T128 H8 hd128 155 -> 105 us, hd64 60 -> 49.)
+        // registers: B64 T128 H8 hd128 155 -> 109 us, hd64 60 -> 50.)
         const int qr = q0 + (lane & 31);
         const int64_t at = (int64_t)(!EX || qr < T ? qr : T - 1) * H;
         if (lane < 32) {
@@ -587,9 +587,9 @@ __device__ __forceinline__ void dkv_tiles(f32x16 (&dka)[HD / 32], f32x16 (&dva)[
 
 // OCC: workgroups per CU the registers allow.  At hd 128 one per CU (all of
 // both accumulators, both fragments and their loads in registers) is faster
-// while each CU has no more than one (B4 T512 H4: 39 against 44 us), two with a
-// few spilled registers beyond that (B32 T64 H8: 34 against 39, B16 T2048 H4:
-// 1380 against 1720).
+// while each CU has no more than one (B4 T512 H4 window 256: 35 against 38 us,
+// B1 T2048 H4: 160 against 207), two with 32 spilled registers beyond that
+// (B24 T64 H8: 26 against 32, B16 T2048 H4: 1061 against 1480).
 template <int HD, int OCC>
 __global__ __launch_bounds__(kThreads, OCC) void attn_dkv_k(float* dk, float* dv, const float* qp, const float* kp,
                                                      const float* vp, const float* dop, const float* lse,
