@@ -1712,10 +1712,10 @@ static inline bool overlaps(const void* a, size_t abytes, const void* b, size_t 
 }
 
 // The bf16-compute kernels take dimensions in multiples of 8 and 16-byte
-// aligned operands.  Other bf16 calls (and fp32 ones with an extent below 8) run the same kernels on zero-padded copies
-// in the workspace (the padding adds zero products only) and copy the valid
-// region back: the tail path of the reference's bounds-checked tiles
-// (ops.mojo:150-168).
+// aligned operands.  Other bf16 calls (and fp32 ones with an extent below 8) run
+// the same kernels on zero-padded copies in the workspace (the padding adds zero
+// products only) and copy the valid region back: the tail path of the
+// reference's bounds-checked tiles (ops.mojo:150-168).
 static bool gemm_direct(const void* C, const void* A, const void* B, int64_t M, int64_t N, int64_t K) {
     return ((M | N | K) & 7) == 0 &&
            ((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(B) | reinterpret_cast<uintptr_t>(C)) & 15) == 0;
